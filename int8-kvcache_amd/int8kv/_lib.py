@@ -129,6 +129,20 @@ def bind(path: Path) -> ctypes.CDLL:
     ]
     lib.int8kv_argmax_rows.restype = ctypes.c_int
     lib.int8kv_argmax_rows.argtypes = [_vp, i64, i64, i64, _vp, _vp]
+    # csrc/skinny_linear.h (the decode loop's own products, not part of the public C ABI)
+    lib.int8kv_skinny_linear_ok.restype = i32
+    lib.int8kv_skinny_linear_ok.argtypes = [i64, i64, i64]
+    lib.int8kv_skinny_linear_workspace_bytes.restype = i64
+    lib.int8kv_skinny_linear_workspace_bytes.argtypes = [i64, i64, i64]
+    lib.int8kv_skinny_linear.restype = ctypes.c_int
+    lib.int8kv_skinny_linear.argtypes = [_vp, i64, i64, i64, _vp, i64, i64, _vp, _vp, i64, _vp,
+                                         i64, _vp]
+    lib.int8kv_skinny_linear_silu_mul.restype = ctypes.c_int
+    lib.int8kv_skinny_linear_silu_mul.argtypes = [_vp, i64, i64, i64, _vp, i64, i64, _vp, i64, _vp]
+    lib.int8kv_skinny_linear_add_rms_norm.restype = ctypes.c_int
+    lib.int8kv_skinny_linear_add_rms_norm.argtypes = [
+        _vp, i64, i64, i64, _vp, i64, i64, _vp, i64, _vp, _vp, i64, f32, _vp, i64, _vp,
+    ]
     lib.int8kv_version.restype = ctypes.c_char_p
     lib.int8kv_version.argtypes = []
     # include/int8kv_probe.h (measurement only: bench.py --ceiling and --cold)

@@ -232,6 +232,68 @@ def hip_silu_mul(gate_up: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def _linear_args(x: torch.Tensor, w: torch.Tensor) -> tuple:
+    _bf16_rows(x, "x")
+    _bf16_rows(w, "w")
+    assert x.shape[1] == w.shape[1] and x.device == w.device
+    return x.data_ptr(), x.shape[0], x.shape[1], x.stride(0), w.data_ptr()
+
+
+def skinny_linear_ok(rows: int, w: torch.Tensor) -> bool:
+    """Whether hip_linear and its fused forms take ``rows`` activation rows times w [n, k]^T."""
+    return (w.dtype == torch.bfloat16 and w.stride(-1) == 1 and w.data_ptr() % 16 == 0
+            and w.stride(0) % 8 == 0 and w.stride(0) >= w.shape[1]
+            and bool(_lib.load().int8kv_skinny_linear_ok(rows, w.shape[1], w.shape[0])))
+
+
+def linear_workspace_bytes(rows: int, w: torch.Tensor) -> int:
+    """Bytes of the ``workspace`` that hip_linear and hip_linear_add_rms_norm take for w."""
+    return _lib.load().int8kv_skinny_linear_workspace_bytes(rows, w.shape[1], w.shape[0])
+
+
+def hip_linear(x: torch.Tensor, w: torch.Tensor, bias: torch.Tensor | None, out: torch.Tensor,
+               workspace: torch.Tensor) -> torch.Tensor:
+    """out = x w^T + bias (bf16, fp32 sums) for at most 32 rows of x (skinny_linear_ok)."""
+    _bf16_rows(out, "out")
+    assert out.shape == (x.shape[0], w.shape[0])
+    if bias is not None:
+        assert bias.dtype == torch.bfloat16 and bias.numel() == w.shape[0]
+        bias = bias.contiguous()
+    status = _lib.load().int8kv_skinny_linear(
+        *_linear_args(x, w), w.shape[0], w.stride(0), None if bias is None else bias.data_ptr(),
+        out.data_ptr(), out.stride(0), workspace.data_ptr(), workspace.numel(),
+        _lib.stream_handle(x.device))
+    _lib.check(status, "int8kv_skinny_linear")
+    return out
+
+
+def hip_linear_silu_mul(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
+    """hip_linear by w_gate_up [2 ffn, k] and hip_silu_mul in one launch, with the same results."""
+    _bf16_rows(out, "out")
+    assert w_gate_up.shape[0] == 2 * out.shape[1] and x.shape[0] == out.shape[0]
+    status = _lib.load().int8kv_skinny_linear_silu_mul(
+        *_linear_args(x, w_gate_up), out.shape[1], w_gate_up.stride(0), out.data_ptr(),
+        out.stride(0), _lib.stream_handle(x.device))
+    _lib.check(status, "int8kv_skinny_linear_silu_mul")
+    return out
+
+
+def hip_linear_add_rms_norm(x: torch.Tensor, w: torch.Tensor, residual: torch.Tensor,
+                            weight: torch.Tensor, out: torch.Tensor, eps: float,
+                            workspace: torch.Tensor) -> torch.Tensor:
+    """hip_linear by w and hip_add_rms_norm(residual, that, weight, out), with the same roundings."""
+    _bf16_rows(residual, "residual")
+    _bf16_rows(out, "out")
+    assert residual.shape == out.shape == (x.shape[0], w.shape[0])
+    assert weight.is_contiguous() and weight.dtype == torch.bfloat16 and weight.numel() == w.shape[0]
+    status = _lib.load().int8kv_skinny_linear_add_rms_norm(
+        *_linear_args(x, w), w.shape[0], w.stride(0), residual.data_ptr(), residual.stride(0),
+        weight.data_ptr(), out.data_ptr(), out.stride(0), eps, workspace.data_ptr(),
+        workspace.numel(), _lib.stream_handle(x.device))
+    _lib.check(status, "int8kv_skinny_linear_add_rms_norm")
+    return out
+
+
 @dataclass
 class LayerWeights:
     ln1: torch.Tensor
@@ -438,6 +500,15 @@ class DecodeLoop:
         self.resid = torch.empty(B, shape.hidden, dtype=torch.bfloat16, device=dev)
         self.normed = torch.empty_like(self.resid)
         self.act = torch.empty(B, shape.ffn, dtype=torch.bfloat16, device=dev)
+        # Buffers of the step's products where the library's weight-streaming kernels take them.
+        H, n_attn = shape.hidden, shape.q_heads * shape.head_dim
+        self.qkv = self.partials = None
+        sizes = [(H, shape.qkv_width), (n_attn, H), (H, 2 * shape.ffn), (shape.ffn, H), (H, shape.vocab)]
+        if all(lib.int8kv_skinny_linear_ok(B, k, n) for k, n in sizes) and shape.ffn % 8 == 0 and H <= 4096:
+            self.qkv = torch.empty(B, shape.qkv_width, dtype=torch.bfloat16, device=dev)
+            self.partials = torch.empty(
+                max(lib.int8kv_skinny_linear_workspace_bytes(B, k, n) for k, n in sizes),
+                dtype=torch.uint8, device=dev)
         self.graph = None
 
     # -- prefill --------------------------------------------------------------------------------
@@ -489,6 +560,10 @@ class DecodeLoop:
         return first
 
     # -- decode ---------------------------------------------------------------------------------
+    def _skinny(self, *weights: torch.Tensor) -> bool:
+        """Whether the step's products by these weights run on the library's kernels (else torch's)."""
+        return self.partials is not None and all(skinny_linear_ok(self.batch, w) for w in weights)
+
     def _step(self) -> None:
         """One greedy step for every sequence: reads/writes only the device state buffers."""
         shape, B = self.shape, self.batch
@@ -501,7 +576,11 @@ class DecodeLoop:
         torch.index_select(self.w.embed, 0, self.tokens, out=x)
         hip_add_rms_norm(x, None, self.w.layers[0].ln1, h, shape.rms_eps)
         for l, lw in enumerate(self.w.layers):
-            qkv = F.linear(h, lw.wqkv, lw.bqkv)
+            skinny = self._skinny(lw.wqkv, lw.wo, lw.w_gate_up, lw.w_down)
+            if skinny:
+                qkv = hip_linear(h, lw.wqkv, lw.bqkv, self.qkv, self.partials)
+            else:
+                qkv = F.linear(h, lw.wqkv, lw.bqkv)
             if FUSED_STEP:
                 self.cache.rotary_write(l, qkv, pos, self.cos, self.sin, self.block_tables)
                 q, _, _ = _split_qkv(qkv, shape)
@@ -510,11 +589,20 @@ class DecodeLoop:
                 q, k, v = _split_qkv(qkv, shape)
                 self.cache.write(l, k, v, slots)
             self.cache.attend(l, q, self.block_tables, self.seq_lens, self.attn_out, self.workspace)
-            hip_add_rms_norm(x, F.linear(self.attn_out.view(B, Hq * D), lw.wo), lw.ln2, h, shape.rms_eps)
-            hip_silu_mul(F.linear(h, lw.w_gate_up), self.act)
+            attn = self.attn_out.view(B, Hq * D)
             nxt = self.w.layers[l + 1].ln1 if l + 1 < L else self.w.ln_f
-            hip_add_rms_norm(x, F.linear(self.act, lw.w_down), nxt, h, shape.rms_eps)
-        torch.mm(h, self.w.lm_head.t(), out=self.logits)
+            if skinny:
+                hip_linear_add_rms_norm(attn, lw.wo, x, lw.ln2, h, shape.rms_eps, self.partials)
+                hip_linear_silu_mul(h, lw.w_gate_up, self.act)
+                hip_linear_add_rms_norm(self.act, lw.w_down, x, nxt, h, shape.rms_eps, self.partials)
+            else:
+                hip_add_rms_norm(x, F.linear(attn, lw.wo), lw.ln2, h, shape.rms_eps)
+                hip_silu_mul(F.linear(h, lw.w_gate_up), self.act)
+                hip_add_rms_norm(x, F.linear(self.act, lw.w_down), nxt, h, shape.rms_eps)
+        if self._skinny(self.w.lm_head):
+            hip_linear(h, self.w.lm_head, None, self.logits, self.partials)
+        else:
+            torch.mm(h, self.w.lm_head.t(), out=self.logits)
         if FUSED_STEP:
             hip_argmax_rows(self.logits, self.tokens)
         else:

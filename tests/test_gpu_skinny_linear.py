@@ -1,0 +1,99 @@
+"""The decode step's products (csrc/skinny_linear.hip) against float64, and their fused forms
+against the separate kernels bit for bit.
+
+Bound of a product: fp32 sums of K exact bf16 products in any order are within K 2^-24 sum|x w| of
+the exact sum, and the bf16 result within half a spacing (2^-8 relative, safely) of that.
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from int8kv import decode_loop as DL
+
+pytestmark = pytest.mark.gpu
+
+# One block of K; slots of unequal length (24 blocks on 8 waves, 41 on 8); eight full slots; K split
+# over groups of workgroups (65 blocks, and the 18944-wide down projection's 296); row blocks
+# below, at and above one per compute unit.
+SHAPES = [(64, 16), (512, 2048), (1536, 48), (2624, 4112), (4096, 4096), (4160, 64), (18944, 3584)]
+
+
+def _inputs(rows, k, n, dev, seed):
+    g = torch.Generator(device=dev).manual_seed(seed)
+    x = torch.randn(rows, k, generator=g, device=dev).to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=g, device=dev) * 0.05).to(torch.bfloat16)
+    b = torch.randn(n, generator=g, device=dev).to(torch.bfloat16)
+    work = torch.empty(max(DL.linear_workspace_bytes(rows, w), 16), dtype=torch.uint8, device=dev)
+    return x, w, b, work
+
+
+@pytest.mark.parametrize("rows", [1, 15, 16, 17, 32])
+@pytest.mark.parametrize("k,n", SHAPES)
+def test_linear_matches_float64(cuda, rows, k, n):
+    x, w, b, work = _inputs(rows, k, n, cuda, rows + k)
+    out = torch.full((rows + 1, n), float("nan"), dtype=torch.bfloat16, device=cuda)
+    for bias in (None, b):
+        DL.hip_linear(x, w, bias, out[:rows], work)
+        ref = x.double() @ w.double().t() + (0 if bias is None else bias.double())
+        mass = x.double().abs() @ w.double().abs().t()
+        err = (out[:rows].double() - ref).abs()
+        assert (err <= 2.0**-8 * ref.abs() + k * 2.0**-24 * (mass + ref.abs())).all()
+        assert torch.isnan(out[rows]).all(), "a row past x was written"
+
+
+@pytest.mark.parametrize("rows", [1, 16, 32])
+@pytest.mark.parametrize("k,ffn", [(64, 8), (512, 1024), (3584, 2376)])
+def test_linear_silu_mul_equals_the_two_kernels(cuda, rows, k, ffn):
+    x, w, _, work = _inputs(rows, k, 2 * ffn, cuda, 7 * rows + k)
+    gate_up = torch.empty(rows, 2 * ffn, dtype=torch.bfloat16, device=cuda)
+    ref = torch.empty(rows, ffn, dtype=torch.bfloat16, device=cuda)
+    out = torch.empty_like(ref)
+    DL.hip_silu_mul(DL.hip_linear(x, w, None, gate_up, work), ref)
+    DL.hip_linear_silu_mul(x, w, out)
+    assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("rows", [1, 16, 32])
+@pytest.mark.parametrize("k,n", [(512, 512), (3584, 3584), (4160, 64), (18944, 3584), (64, 8192)])
+def test_linear_add_rms_norm_equals_the_two_kernels(cuda, rows, k, n):
+    x, w, b, work = _inputs(rows, k, n, cuda, 11 * rows + k)
+    residual = torch.randn(rows, n, device=cuda).to(torch.bfloat16)
+    ref_res, ref = residual.clone(), torch.empty_like(residual)
+    DL.hip_add_rms_norm(ref_res, DL.hip_linear(x, w, None, torch.empty_like(residual), work), b, ref, 1e-6)
+    out = torch.empty_like(residual)
+    DL.hip_linear_add_rms_norm(x, w, residual, b, out, 1e-6, work)
+    assert torch.equal(residual, ref_res)
+    # The row's sum of squares is added in another order: at most one bf16 step of each rounding.
+    assert ((out.double() - ref.double()).abs() <= 2.0**-6 * ref.double().abs()).all()
+
+
+def test_non_finite_values_stay_in_their_rows_and_columns(cuda):
+    x, w, _, work = _inputs(20, 512, 64, cuda, 3)
+    x[3, 100] = float("nan")
+    w[5, 7] = float("inf")
+    out = DL.hip_linear(x, w, None, torch.empty(20, 64, dtype=torch.bfloat16, device=cuda), work)
+    ref = x.double() @ w.double().t()
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    assert torch.equal(torch.isposinf(out), torch.isposinf(ref))
+    assert torch.equal(torch.isneginf(out), torch.isneginf(ref))
+
+
+def test_what_the_kernels_take(cuda):
+    w = torch.zeros(64, 128, dtype=torch.bfloat16, device=cuda)
+    assert DL.skinny_linear_ok(1, w) and DL.skinny_linear_ok(32, w)
+    assert not DL.skinny_linear_ok(33, w) and not DL.skinny_linear_ok(0, w)
+    assert not DL.skinny_linear_ok(1, w[:, :96]) and not DL.skinny_linear_ok(1, w[:24])
+    assert not DL.skinny_linear_ok(1, w[:, 4:68]) and not DL.skinny_linear_ok(1, w.float())
+
+
+@pytest.mark.parametrize("batch,hidden", [(33, 512), (3, 480)])
+def test_step_falls_back_to_torch_products(cuda, batch, hidden):
+    shape = DL.QwenShape(hidden=hidden, layers=1, q_heads=28, kv_heads=4, head_dim=128, ffn=1024, vocab=2048)
+    weights = DL.random_weights(shape, cuda, seed=1)
+    loop = DL.DecodeLoop(weights, batch, 5, 2, "bf16")
+    assert loop.partials is None
+    loop.prefill(torch.zeros(batch, 5, dtype=torch.int64))
+    loop.step_eager()
+    assert torch.isfinite(loop.logits.float()).all()
