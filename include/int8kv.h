@@ -266,8 +266,8 @@ int int8kv_decode_plan(int query_dtype, int cache_dtype, int64_t batch, int32_t 
  * an output nor stored: 80, 96 and 112 on the 128-wide kernels, for example), block_size a
  * power of two in [16, 65536] (16 and 32 are vLLM's usual values), any integer group =
  * num_q_heads / num_kv_heads with num_kv_heads x ceil(group / 16) <= 65535 (a kv head's query
- * heads are taken 16 at a time, one wave or workgroup per 16: multi-query attention with 64
- * query heads runs 4 waves per kv head).  Other sizes return INT8KV_E_SHAPE.
+ * heads are taken 16 at a time: one wave or workgroup per 16, or, for larger calls in the range
+ * layout at head_dim up to 128, up to 5 such tiles per wave).  Other sizes return INT8KV_E_SHAPE.
  */
 int int8kv_paged_decode(const void* query, int query_dtype, int64_t batch, int32_t num_q_heads,
                         int32_t head_dim, const int64_t query_strides[3], const void* key_cache,

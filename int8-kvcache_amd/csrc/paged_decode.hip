@@ -79,9 +79,13 @@ constexpr int kMaxRangesLimit = 1 << 20;
 constexpr int kSeqStartCost = 2;        // host-side bounds, and 16-bit caches
 constexpr int kSeqStartCostI8 = 4;      // INT8, two tiles in flight
 constexpr int kSeqStartCostI8Deep = 6;  // INT8, four tiles in flight
+// Groups above 16: four waves share a tile's time, so a start is more tile times (71 heads, B =
+// 40 x 4096: 8 units 30.6 us, 14 28.5, 20 28.5, 28 29.2; U[1, 8192] 31.4 / 29.0 / 30.1 / 29.9).
+constexpr int kSeqStartCostWide = 14;
 // Smallest automatic range (see auto_min_tiles).
 constexpr int kMinTilesSmall = 2;
 constexpr int kMinTilesLarge = 4;
+constexpr int kWideMinUnits = 8;  // groups above 16: two tiles for each of a workgroup's four waves
 constexpr int64_t kMaxMergeRanges = 128;  // ranges per sequence the merge takes in 4 rounds
 // Resident decode waves per CU the automatic range count targets: one per SIMD.  Against two
 // per SIMD (the second of which streams ~30 % slower) it measured 3-11 % faster on every
@@ -246,9 +250,29 @@ bool kv_pair_shape(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim) 
   return head_dim == 64 && num_kv_heads % 2 == 0 && num_q_heads / num_kv_heads <= 8;
 }
 
+// MFMA column tiles of 16 query heads per kv head, and the grid's heads (kv heads x tiles).
+int32_t col_tiles(int32_t num_q_heads, int32_t num_kv_heads) {
+  return (num_q_heads / num_kv_heads + kMaxGroup - 1) / kMaxGroup;
+}
+
+int32_t grid_heads(int32_t num_q_heads, int32_t num_kv_heads) {
+  return num_kv_heads * col_tiles(num_q_heads, num_kv_heads);
+}
+
 int32_t auto_ranges(int32_t num_kv_heads, int64_t cu) {
   const int64_t p = cu * kWavesPerCU / num_kv_heads;
   return (int32_t)(p < 1 ? 1 : (p > kMaxRangesLimit ? kMaxRangesLimit : p));
+}
+
+// Automatic range count of a shape: one wave per SIMD for the grid heads (a kv-head pair counts as
+// one); for the wide kernel (paged_decode_wide.h) at least one workgroup per CU.
+int32_t auto_ranges_for(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, bool pair,
+                        int64_t cu) {
+  const int32_t tiles = col_tiles(num_q_heads, num_kv_heads);
+  const int32_t r = auto_ranges(pair ? num_kv_heads / 2 : num_kv_heads * tiles, cu);
+  const int32_t most = wide_most_tiles(padded_head_dim(head_dim));
+  if (tiles == 1 || most == 1) return r;
+  return std::max(r, (int32_t)(cu / (num_kv_heads * ((tiles + most - 1) / most))));
 }
 
 // Per range: 2 x num_q_heads partial records (head_dim + 2 floats each) and the 32-byte
@@ -280,15 +304,6 @@ bool shape_ok(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int32
          head_dim % 16 == 0 && block_size_ok(block_size);
 }
 
-// MFMA column tiles of 16 query heads per kv head, and the grid's heads (kv heads x tiles).
-int32_t col_tiles(int32_t num_q_heads, int32_t num_kv_heads) {
-  return (num_q_heads / num_kv_heads + kMaxGroup - 1) / kMaxGroup;
-}
-
-int32_t grid_heads(int32_t num_q_heads, int32_t num_kv_heads) {
-  return num_kv_heads * col_tiles(num_q_heads, num_kv_heads);
-}
-
 }  // namespace
 
 extern "C" int32_t int8kv_decode_auto_ranges(int32_t num_kv_heads) {
@@ -303,10 +318,8 @@ extern "C" size_t int8kv_decode_workspace_bytes(int32_t num_q_heads, int32_t num
       num_ranges > kMaxRangesLimit)
     return 0;
   if (num_ranges == 0)
-    num_ranges = auto_ranges(kv_pair_shape(num_q_heads, num_kv_heads, head_dim)
-                                 ? num_kv_heads / 2
-                                 : grid_heads(num_q_heads, num_kv_heads),
-                             cu_count());
+    num_ranges = auto_ranges_for(num_q_heads, num_kv_heads, head_dim,
+                                 kv_pair_shape(num_q_heads, num_kv_heads, head_dim), cu_count());
   return workspace_bytes(num_q_heads, num_ranges, padded_head_dim(head_dim));
 }
 
@@ -400,7 +413,8 @@ int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_hea
   const bool kv_pair_ok = kv_pair_shape(num_q_heads, num_kv_heads, head_dim) &&
                           key_head_stride == head_dim && value_head_stride == head_dim;
   const int32_t wave_heads = kv_pair_ok ? num_kv_heads / 2 : hv;  // per range
-  if (num_ranges == 0) num_ranges = auto_ranges(wave_heads, cus);
+  if (num_ranges == 0)
+    num_ranges = auto_ranges_for(num_q_heads, num_kv_heads, head_dim, kv_pair_ok, cus);
   if (scratch_cap > 0 && auto_ranges_req) {
     // The partials of the automatic count may exceed the fixed scratch array (large GQA groups
     // or head_dim 256): take the most ranges it holds instead.
@@ -461,10 +475,42 @@ int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_hea
                   ? 4
                   : 2;
   }
+  // Groups above 16 query heads: the wide kernel, one range per workgroup of four waves and one
+  // workgroup per CU, with as many column tiles per wave as its registers hold, spread evenly
+  // (5 tiles of 16: one wave at head_dim 64, 3 + 2 at 128), or fewer where the workgroups would
+  // otherwise hold under kWideMinUnits units of work each; under that even at two tiles per
+  // wave, and above head_dim 128 (one tile per wave), a wave per column tile as decode_kernel.
+  // 71 query heads on one kv head at 64, INT8, us before -> now (HIP-graph replays): B = 40 x 4096
+  // 41.2 -> 28.5, 40 x U[1, 8192] 43.2 -> 29.0, 8 x 4096 (3 + 2 tiles) 17.2 -> 16.7 (19.6 with 5);
+  // 16-bit cache 40 x 4096 30.0 -> 28.6; at 128: 64 heads on one, 16 x 8192 31.3 -> 27.7; 48 on
+  // two, 64 x U[1, 8192] 53.7 -> 47.9.
+  p.ct = 0;
+  p.launch_ranges = num_ranges;
+  p.launch_min_tiles = min_tiles;
+  const int32_t most = wide_most_tiles(hd);
+  if (p.col_tiles > 1 && !p.group_mode && most > 1) {
+    const int32_t tiles = p.col_tiles;
+    const double units = (double)batch * std::ceil((double)table_width * block_size / tile_tokens);
+    for (int32_t waves = (tiles + most - 1) / most; waves < tiles; ++waves) {
+      const int32_t heads = num_kv_heads * waves;  // workgroups per range
+      if (units * heads < (double)kWideMinUnits * cus) continue;
+      p.ct = (tiles + waves - 1) / waves;
+      p.col_tiles = waves;
+      p.grid_heads = heads;
+      p.depth = 2;
+      p.halves = 1;
+      p.pair_min = 0x7fffffff;
+      if (auto_ranges_req)
+        p.launch_ranges = (int32_t)std::max<int64_t>(1, std::min<int64_t>(num_ranges, cus / heads));
+      if (automatic) p.launch_min_tiles = std::max(min_tiles, kWideMinUnits);
+      break;
+    }
+  }
   // The layout above was chosen with the base charge; the plan itself charges what a sequence
   // start costs at the chosen depth (kSeqStartCost*).  decode_kernel and merge_kernel read the
   // same value, so their range bounds agree.
   if (i8) p.seq_cost = p.depth == 4 ? kSeqStartCostI8Deep : kSeqStartCostI8;
+  if (p.ct > 0) p.seq_cost = kSeqStartCostWide;
   // Four tiles in flight leave no registers for an fp32 query's lo operands: two for those.
   p.launch_depth = p.group_mode ? 2 : (p.depth == 4 && query_dtype != INT8KV_F32 ? 4 : 2);
   // Units of one sequence are at most ceil(table_width x block_size / 32) + seq_cost (lengths are
@@ -475,7 +521,7 @@ int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_hea
   // The merge indexed by range (from descriptors the decode kernel then writes) for batches of
   // at least half the range count, where its grid is the smaller one; below that, the merge
   // indexed by sequence, and no descriptors.
-  p.cut_desc = 2 * batch >= (int64_t)num_ranges;
+  p.cut_desc = 2 * batch >= (int64_t)p.launch_ranges;
   if (p.group_mode) {
     p.merge = p.split > 0 ? kMergeSplit : kMergeNone;
     p.merge_waves = p.split > 0 ? 1 : 0;
@@ -487,7 +533,7 @@ int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_hea
   } else {
     p.merge = kMergeBySequence;
     merge_shape(batch > 0 ? batch : 1, table_width, block_size, tile_tokens, p.seq_cost,
-                min_tiles, num_ranges, &p.merge_waves, &p.merge_fold);
+                p.launch_min_tiles, p.launch_ranges, &p.merge_waves, &p.merge_fold);
   }
   // Non-temporal K/V loads when the call may stream more than kNonTemporalMinBytes: the most it
   // can read is min(pool, batch x table width) blocks of K and V (host-side sizes only).  INT8
@@ -602,8 +648,8 @@ int decode_entry(
   a.group = num_q_heads / num_kv_heads;
   a.col_tiles = hp.col_tiles;
   a.width = (int32_t)table_width;
-  a.max_ranges = hp.num_ranges;
-  a.min_tiles = hp.min_tiles;
+  a.max_ranges = hp.launch_ranges;
+  a.min_tiles = hp.launch_min_tiles;
   a.seq_cost = hp.seq_cost;
   a.quantize_q = (flags & INT8KV_DECODE_QUANTIZE_Q) != 0;
   a.group_mode = hp.group_mode;

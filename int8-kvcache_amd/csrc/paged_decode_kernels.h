@@ -1921,9 +1921,32 @@ struct HostPlan {
   bool pad;             // the cache's head_dim is below hd
   int32_t grid_heads;   // kv heads x col_tiles
   int32_t col_tiles;    // MFMA column tiles of 16 query heads per kv head
+  int32_t ct;           // column tiles per wave (paged_decode_wide.h); 0: one grid head per wave
+  int32_t launch_ranges;  // ranges the kernels run with (num_ranges, or fewer with ct)
+  int32_t launch_min_tiles;
   int64_t cus;
   size_t need;          // workspace bytes
 };
+
+// Most column tiles of 16 query heads that one wave of the wide range kernel holds
+// (paged_decode_wide.h): its accumulators (HD / 4 registers a tile) and query operands (HD / 8,
+// twice that for an fp32 query) next to two tiles of K/V in the 512 registers of a one-wave SIMD,
+// and four waves' states in 160 KB of LDS.  At 256 a second tile spills 0.5-1 KB per lane.
+constexpr int wide_most_tiles(int hd) { return hd == 64 ? 5 : hd == 128 ? 3 : 1; }
+
+// The wide range kernel per cache type (paged_decode_wide_<type>.hip).
+int launch_wide_int8(const DecodeArgs& a, const HostPlan& hp, int query_dtype, hipStream_t s);
+int launch_wide_int8_pad(const DecodeArgs& a, const HostPlan& hp, int query_dtype, hipStream_t s);
+int launch_wide_bf16(const DecodeArgs& a, const HostPlan& hp, int query_dtype, hipStream_t s);
+int launch_wide_fp16(const DecodeArgs& a, const HostPlan& hp, int query_dtype, hipStream_t s);
+
+template <int CACHE, int QT>
+inline int launch_wide(const DecodeArgs& a, const HostPlan& hp, hipStream_t s) {
+  const int q = QT;  // the dtype codes are the template's tags
+  if constexpr (CACHE == kI8) return hp.pad ? launch_wide_int8_pad(a, hp, q, s) : launch_wide_int8(a, hp, q, s);
+  if constexpr (CACHE == kBF16) return launch_wide_bf16(a, hp, q, s);
+  return launch_wide_fp16(a, hp, q, s);
+}
 
 // PAD: head_dim below HD (the kernels' padded instances; the plan keeps them to one range per
 // workgroup with two tiles in flight and no kv-head pairs).
@@ -1959,7 +1982,10 @@ int launch(const DecodeArgs& a, const HostPlan& hp, uint32_t flags, hipStream_t 
     }
     return INT8KV_OK;
   }
-  if (flags & INT8KV_DECODE_MAIN) {
+  if ((flags & INT8KV_DECODE_MAIN) && hp.ct > 0) {
+    const int e = launch_wide<CACHE, QT>(a, hp, s);
+    if (e != 0) return e;
+  } else if (flags & INT8KV_DECODE_MAIN) {
     dim3 grid((unsigned)((a.max_ranges + a.halves - 1) / a.halves), (unsigned)(hv / W));
     if constexpr (HD == 64 && !PAD) {
       if (a.kv_pair)

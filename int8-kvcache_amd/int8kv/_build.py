@@ -21,10 +21,14 @@ LIB_PATH = PKG_DIR / "libint8kv.so"
 
 # The paged decode's kernels compile per cache type in parallel (paged_decode_<type>.hip and, for
 # head_dims below the kernels' 64 / 128 / 256, paged_decode_<type>_pad.hip, from
-# paged_decode_kernels.h); paged_decode.hip is its host side.
+# paged_decode_kernels.h; for GQA groups above 16, paged_decode_wide_<type>.hip, from
+# paged_decode_wide.h); paged_decode.hip is its host side.
 SOURCES = ["cache_write.hip", "paged_decode.hip", "paged_decode_int8.hip", "paged_decode_bf16.hip",
            "paged_decode_fp16.hip", "paged_decode_int8_pad.hip", "paged_decode_bf16_pad.hip",
-           "paged_decode_fp16_pad.hip", "decode_loop_ops.hip", "skinny_linear.hip", "read_probe.hip"]
+           "paged_decode_fp16_pad.hip", "paged_decode_wide_int8.hip",
+           "paged_decode_wide_int8_pad.hip", "paged_decode_wide_bf16.hip",
+           "paged_decode_wide_fp16.hip", "decode_loop_ops.hip", "skinny_linear.hip",
+           "read_probe.hip"]
 # The torch extension over the C ABI (host code only; torch headers, linked to libint8kv.so).
 EXT_SOURCE = "torch_ops.cpp"
 EXT_NAME = "_int8kv_torch"

@@ -207,3 +207,40 @@ def test_write_then_decode(cuda):
     out = int8kv.int8_paged_attention(q, kc, vc, bt, sl, ks, vs)
     torch.cuda.synchronize()
     _check(out, oracle_int8(c), "write then decode d=80")
+
+
+# Groups above 16 with enough work for the kernel that holds several column tiles per wave: 2, 3,
+# 4 and 5 tiles at head_dim 64, 2 and 3 at 128 (a last tile of one head; kv heads of two waves),
+# padded head_dims, and sequences of 0 to 2 segments per range.
+WIDE = [(17, 1, 64), (48, 1, 64), (64, 1, 64), (71, 1, 64), (96, 1, 64), (66, 2, 128), (48, 1, 128),
+        (71, 1, 128), (40, 2, 96), (33, 1, 48)]
+WIDE_LENS = [0, 1, 33, 9000, 255, 4097, 31, 64, 12345, 2200, 0, 700] + [1500] * 10
+
+
+@pytest.mark.parametrize("cache", ["int8", "bf16", "fp16"])
+@pytest.mark.parametrize("hq,hkv,d", WIDE)
+def test_groups_above_16_several_tiles_per_wave(cuda, hq, hkv, d, cache):
+    c = decode_case(WIDE_LENS, seed=hq * 5 + d, hq=hq, hkv=hkv, head_dim=d, extra_blocks=7)
+    t = to_dev(c, cuda)
+    q, kc, vc, bt, sl, ks, vs = t
+    if cache == "int8":
+        full, out = _decode_auto(*t)
+        _check(out, oracle_int8(c), f"{hq}/{hkv} d={d} auto")
+        _untouched(full, d, f"{hq}/{hkv} d={d} auto")
+        out = ranges_call(t, cuda, splits=3)
+        _check(out, oracle_int8(c), f"{hq}/{hkv} d={d} ranges x3")
+        out = int8kv.int8_paged_attention(q.float(), kc, vc, bt, sl, ks, vs)
+        assert _check(out, oracle_int8(c), f"{hq}/{hkv} d={d} fp32 query") <= 1e-3
+        for query in (q, q.float()):  # quantised: the same integer scores from either dtype
+            out = int8kv.int8_paged_attention(query, kc, vc, bt, sl, ks, vs, quantize_q=True)
+            ref = O.paged_attention_ref(c.query.float().numpy(), c.kc, c.vc, c.block_tables.numpy(),
+                                        c.seq_lens.numpy(), c.k_scale.numpy(), c.v_scale.numpy(),
+                                        quantize_q=True)
+            _check(out, ref, f"{hq}/{hkv} d={d} quantize_q")
+        return
+    k_cpu, v_cpu = bf16_caches(c, torch.bfloat16 if cache == "bf16" else torch.float16)
+    ref = O.paged_attention_ref(c.query.float().numpy(), k_cpu.float().numpy(),
+                                v_cpu.float().numpy(), c.block_tables.numpy(), c.seq_lens.numpy())
+    out = int8kv.bf16_paged_attention(q, k_cpu.to(cuda), v_cpu.to(cuda), bt, sl)
+    assert (out[0] == 0).all() and (out[10] == 0).all()
+    _check(out, ref, f"{hq}/{hkv} d={d} {cache}")
