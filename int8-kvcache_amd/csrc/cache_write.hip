@@ -7,7 +7,8 @@
 // zero (:59-63); this kernel deliberately does not.  The scale is clamped to >= 1e-6 as the
 // Triton kernel does (:50-51); calibrated scales already satisfy that (scripts/04 :55-65).
 //
-// Mapping (wide kernels, head_dim % 16 == 0 and 16-byte aligned cache rows): grid.y = kv head,
+// Mapping of 16-bit sources (wide kernels, head_dim % 16 == 0 and 16-byte aligned cache rows; fp32
+// sources and small calls take the row kernels, one 16-byte load per lane): grid.y = kv head,
 // one lane owns 16 consecutive head_dim elements of one (token, head) row of both K and V --
 // 32-byte source loads, 16-byte cache stores, 8 lanes per 128-element row.  The slot is read
 // first, so skipped rows cost no source bytes.  Sources are read and caches written with the
@@ -107,6 +108,7 @@ __global__ __launch_bounds__(256) void cache_write_kernel(WriteArgs a) {
 
 
 // ------------------------------------------------------------------ wide kernels (16 per lane)
+// 16-bit sources.
 template <bool NT>
 __device__ __forceinline__ u32x4 ld16(const char* p) {
   if constexpr (NT)
@@ -115,27 +117,14 @@ __device__ __forceinline__ u32x4 ld16(const char* p) {
     return *reinterpret_cast<const u32x4*>(p);
 }
 
-// 16 consecutive elements of type DT at p (16-byte aligned), widened to fp32, non-temporal.
+// 16 consecutive 16-bit elements at p (16-byte aligned), widened to fp32, non-temporal.
 template <int DT>
 __device__ __forceinline__ void load16_f32(const char* p, float (&x)[16]) {
-  if constexpr (DT == kF32) {
-    // Typed f32x4 loads: element reads of a bit-cast u32x4 were miscompiled here (repeated
-    // elements), as in the decode kernel's fp32 query path.
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const f32x4 w = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p + 16 * j));
-      x[4 * j + 0] = w[0];
-      x[4 * j + 1] = w[1];
-      x[4 * j + 2] = w[2];
-      x[4 * j + 3] = w[3];
-    }
-  } else {
+  for (int j = 0; j < 2; ++j) {
+    const u32x4 w = ld16<true>(p + 16 * j);
 #pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const u32x4 w = ld16<true>(p + 16 * j);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) unpack2<DT>(w[i], x[8 * j + 2 * i], x[8 * j + 2 * i + 1]);
-    }
+    for (int i = 0; i < 4; ++i) unpack2<DT>(w[i], x[8 * j + 2 * i], x[8 * j + 2 * i + 1]);
   }
 }
 
@@ -173,6 +162,90 @@ __global__ __launch_bounds__(256) void cache_write16_kernel(WriteArgs a) {
   const u32x4 vq = {wv[0], wv[1], wv[2], wv[3]};
   store16_nt(a.kc + blk * a.kc_sb + off * a.kc_ss + h * a.kc_sh + 16 * dv, kq);
   store16_nt(a.vc + blk * a.vc_sb + off * a.vc_ss + h * a.vc_sh + 16 * dv, vq);
+}
+
+// ------------------------------------------------------------------ row kernels (one load per lane)
+// One 16-byte load of K and of V per lane: a row's adjacent lanes read one contiguous run, whole
+// 128-byte lines per instruction, and store its codes as whole lines too.
+//   * fp32 sources always: with 16 elements per lane each of a lane's four loads met every fourth
+//     16-byte piece of its lines (40,000 x 4 x 128: static 52.9 -> 37.6 us, dynamic 58.8 -> 46.0;
+//     200,000: 243 -> 182 and 197 us).  Two or four pieces per lane: static 1-3 % slower, dynamic
+//     3-5 % faster above 100 MB, both up to twice the time at 32 tokens.
+//   * 16-bit sources below kRowKernelElements: with 16 elements per lane those calls leave SIMDs
+//     without a wave (32 tokens x 4 x 128 static 2.87 -> 2.66 us, dynamic 3.86 -> 3.37; 256 x 8 x
+//     128 dynamic 4.28 -> 3.60); above, half the index work per element wins (16,384 x 4 x 128
+//     static 13.1 vs 11.5 us; 100,003 x 8 x 128 dynamic 128 vs 117 us).
+constexpr int64_t kRowKernelElements = 1 << 20;  // tokens x kv heads x head_dim
+
+template <int SRC>
+constexpr int kPiece = SRC == kF32 ? 4 : 8;  // elements of a load
+
+template <int SRC>
+__device__ __forceinline__ void load_piece(const char* p, float (&x)[kPiece<SRC>]) {
+  if constexpr (SRC == kF32) {
+    // Typed f32x4 load: element reads of a bit-cast u32x4 were miscompiled here (repeated
+    // elements), as in the decode kernel's fp32 query path.
+    const f32x4 w = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = w[i];
+  } else {
+    const u32x4 w = ld16<true>(p);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) unpack2<SRC>(w[i], x[2 * i], x[2 * i + 1]);
+  }
+}
+
+template <int W>
+__device__ __forceinline__ void store_codes(int8_t* p, const uint32_t (&w)[W]) {
+  if constexpr (W == 1)
+    __builtin_nontemporal_store(w[0], reinterpret_cast<uint32_t*>(p));
+  else
+    __builtin_nontemporal_store(u32x2{w[0], w[1]}, reinterpret_cast<u32x2*>(p));
+}
+
+// This lane's piece: token, kv head, piece of the head's row.  Head-major (TM false): grid.y is the
+// kv head.  Token-major: a token's kv heads follow one another, 1 << lpt_shift lanes per token (kv
+// heads and pieces per row powers of two).
+template <bool TM>
+__device__ __forceinline__ void row_piece(const WriteArgs& a, int lpr_shift, int lpt_shift, uint32_t& t,
+                                          int& h, int& dv) {
+  const uint32_t idx = blockIdx.x * 256u + threadIdx.x;
+  if constexpr (TM) {
+    t = idx >> lpt_shift;
+    const uint32_t w = idx & ((1u << lpt_shift) - 1u);
+    h = (int)(w >> lpr_shift);
+    dv = (int)(w & ((1u << lpr_shift) - 1u));
+  } else {
+    const uint32_t lpr = (uint32_t)a.vecs_per_row;
+    t = div_uniform(idx, lpr);
+    h = blockIdx.y;
+    dv = (int)(idx - t * lpr);
+  }
+}
+
+template <int SRC, bool TM>
+__global__ __launch_bounds__(256) void cache_write_rows_kernel(WriteArgs a, int lpr_shift, int lpt_shift) {
+  constexpr int P = kPiece<SRC>;
+  constexpr int esize = SRC == kF32 ? 4 : 2;
+  uint32_t t;
+  int h, dv;
+  row_piece<TM>(a, lpr_shift, lpt_shift, t, h, dv);
+  if ((int64_t)t >= a.num_tokens) return;
+  // Slot and source bytes together below the Infinity Cache's size, the slot first above it
+  // (token-major there): as in the 16-element kernels.
+  const int64_t slot = load_index(a.slots, t, a.slots_is64);
+  if (TM && (slot < 0 || slot >= a.capacity)) return;
+  float x[P], y[P];
+  load_piece<SRC>(a.key + ((int64_t)t * a.k_st + h * a.k_sh + P * dv) * esize, x);
+  load_piece<SRC>(a.value + ((int64_t)t * a.v_st + h * a.v_sh + P * dv) * esize, y);
+  if (slot < 0 || slot >= a.capacity) return;
+  int64_t blk, off;
+  slot_block(a, slot, blk, off);
+  uint32_t wk[P / 4], wv[P / 4];
+  quantise<P, false>(x, quant_scale(fmaxf(a.k_scale[h], 1e-6f)), wk);
+  quantise<P, false>(y, quant_scale(fmaxf(a.v_scale[h], 1e-6f)), wv);
+  store_codes(a.kc + blk * a.kc_sb + off * a.kc_ss + h * a.kc_sh + P * dv, wk);
+  store_codes(a.vc + blk * a.vc_sb + off * a.vc_ss + h * a.vc_sh + P * dv, wv);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -388,6 +461,75 @@ __global__ __launch_bounds__(256) void dynamic_write16_tm_kernel(DynWriteArgs d,
   }
 }
 
+// Row kernel of the dynamic write: vecs_per_row = head_dim / kPiece is a power of two of at most
+// 64, so a wave holds whole rows and the absmax butterfly stays inside the row.  Token-major, the
+// scales of four consecutive heads (when their lanes share a wave: vec_scales) leave in one
+// 16-byte store.
+template <int SRC, bool TM>
+__global__ __launch_bounds__(256) void dynamic_write_rows_kernel(DynWriteArgs d, int lpr_shift, int lpt_shift) {
+  const WriteArgs& a = d.w;
+  constexpr int P = kPiece<SRC>;
+  constexpr int esize = SRC == kF32 ? 4 : 2;
+  uint32_t t;
+  int h, dv;
+  row_piece<TM>(a, lpr_shift, lpt_shift, t, h, dv);
+  // Every lane takes part in the exchanges; those past the last token and (token-major) of skipped
+  // rows hold zeros.
+  int64_t slot = -1;
+  float x[P], y[P];
+#pragma unroll
+  for (int i = 0; i < P; ++i) x[i] = y[i] = 0.0f;
+  if ((int64_t)t < a.num_tokens) {
+    slot = load_index(a.slots, t, a.slots_is64);
+    if (slot >= a.capacity) slot = -1;
+    load_piece<SRC>(a.key + ((int64_t)t * a.k_st + h * a.k_sh + P * dv) * esize, x);
+    load_piece<SRC>(a.value + ((int64_t)t * a.v_st + h * a.v_sh + P * dv) * esize, y);
+  }
+  float km = 0.0f, vm = 0.0f;
+#pragma unroll
+  for (int i = 0; i < P; ++i) {
+    km = fmaxf(km, fabsf(x[i]));
+    vm = fmaxf(vm, fabsf(y[i]));
+  }
+  const int lpr = 1 << lpr_shift;
+  for (int o = 1; o < lpr; o <<= 1) {
+    km = fmaxf(km, __shfl_xor(km, o));
+    vm = fmaxf(vm, __shfl_xor(vm, o));
+  }
+  const float ks = fmaxf(km / 127.0f, 1e-6f);
+  const float vs = fmaxf(vm / 127.0f, 1e-6f);
+  const bool vec = TM && d.vec_scales;
+  f32x4 k4 = {ks, 0.f, 0.f, 0.f}, v4 = {vs, 0.f, 0.f, 0.f};
+  if (vec) {
+    const int lane = threadIdx.x % kWave;
+#pragma unroll
+    for (int i = 1; i < 4; ++i) {
+      k4[i] = __shfl(ks, lane + i * lpr);
+      v4[i] = __shfl(vs, lane + i * lpr);
+    }
+  }
+  if (slot < 0) return;
+  int64_t blk, off;
+  slot_block(a, slot, blk, off);
+  uint32_t wk[P / 4], wv[P / 4];
+  quantise<P, true>(x, quant_scale(ks), wk);
+  quantise<P, true>(y, quant_scale(vs), wv);
+  store_codes(a.kc + blk * a.kc_sb + off * a.kc_ss + h * a.kc_sh + P * dv, wk);
+  store_codes(a.vc + blk * a.vc_sb + off * a.vc_ss + h * a.vc_sh + P * dv, wv);
+  if (dv != 0) return;
+  float* kp = d.ksc + blk * d.ksc_sb + off * d.ksc_ss + h * d.ksc_sh;
+  float* vp = d.vsc + blk * d.vsc_sb + off * d.vsc_ss + h * d.vsc_sh;
+  if (vec) {
+    if ((h & 3) == 0) {
+      *reinterpret_cast<f32x4*>(kp) = k4;
+      *reinterpret_cast<f32x4*>(vp) = v4;
+    }
+  } else {
+    *kp = ks;
+    *vp = vs;
+  }
+}
+
 }  // namespace int8kv
 
 using namespace int8kv;
@@ -427,6 +569,45 @@ constexpr double kInfinityCacheBytes = 256.0 * 1024 * 1024;
 bool static_token_major(int64_t num_tokens, int32_t num_kv_heads, int32_t head_dim,
                         int64_t src_esize) {
   return (double)num_tokens * num_kv_heads * head_dim * (2.0 * src_esize + 2.0) > kInfinityCacheBytes;
+}
+
+bool power_of_two(int64_t n) { return n > 0 && (n & (n - 1)) == 0; }
+
+// Grid of a row kernel for `lpr` pieces per row (tm: the token-major map); false when the call's
+// pieces overflow its 32-bit index.
+bool rows_grid(const WriteArgs& a, bool tm, dim3* grid) {
+  const int64_t pieces = a.num_tokens * a.vecs_per_row * (tm ? a.num_kv_heads : 1);
+  if (pieces > 0x7fffff00LL) return false;
+  *grid = dim3((unsigned)((pieces + 255) / 256), tm ? 1u : (unsigned)a.num_kv_heads);
+  return true;
+}
+
+template <int SRC>
+int launch_rows(const WriteArgs& a, bool tm, dim3 grid, hipStream_t s) {
+  if (tm)
+    hipLaunchKernelGGL((cache_write_rows_kernel<SRC, true>), grid, dim3(256), 0, s, a,
+                       __builtin_ctz((unsigned)a.vecs_per_row),
+                       __builtin_ctz((unsigned)(a.vecs_per_row * a.num_kv_heads)));
+  else
+    hipLaunchKernelGGL((cache_write_rows_kernel<SRC, false>), grid, dim3(256), 0, s, a, 0, 0);
+  return (int)hipGetLastError();
+}
+
+template <int SRC>
+int launch_dynamic_rows(const DynWriteArgs& d, bool tm, dim3 grid, hipStream_t s) {
+  const int lpr_shift = __builtin_ctz((unsigned)d.w.vecs_per_row);
+  if (tm)
+    hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, true>), grid, dim3(256), 0, s, d, lpr_shift,
+                       __builtin_ctz((unsigned)(d.w.vecs_per_row * d.w.num_kv_heads)));
+  else
+    hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, false>), grid, dim3(256), 0, s, d, lpr_shift, 0);
+  return (int)hipGetLastError();
+}
+
+// Whether a call takes the row kernels.
+bool use_rows(int src_dtype, int64_t num_tokens, int32_t num_kv_heads, int32_t head_dim) {
+  return src_dtype == INT8KV_F32 ||
+         (double)num_tokens * num_kv_heads * head_dim < (double)kRowKernelElements;
 }
 
 // Validates the arguments shared by the static and the dynamic write and fills WriteArgs.
@@ -509,18 +690,27 @@ extern "C" int int8kv_cache_write(const void* key, const void* value, int src_dt
   a.v_scale = v_scale;
   hipStream_t s = static_cast<hipStream_t>(stream);
 
-  if (wide_ok(key_cache, value_cache, key_cache_strides, value_cache_strides, num_tokens,
-              num_kv_heads, head_dim)) {
+  const bool wide = wide_ok(key_cache, value_cache, key_cache_strides, value_cache_strides,
+                            num_tokens, num_kv_heads, head_dim);
+  const int64_t src_esize = src_dtype == INT8KV_F32 ? 4 : 2;
+  const bool streams = static_token_major(num_tokens, num_kv_heads, head_dim, src_esize);
+  if (wide && use_rows(src_dtype, num_tokens, num_kv_heads, head_dim)) {
+    WriteArgs r = a;
+    r.vecs_per_row = (int32_t)(head_dim * src_esize / 16);
+    const bool tm = streams && power_of_two(num_kv_heads) && power_of_two(r.vecs_per_row);
+    dim3 grid;
+    if (rows_grid(r, tm, &grid))
+      return src_dtype == INT8KV_F32   ? launch_rows<kF32>(r, tm, grid, s)
+             : src_dtype == INT8KV_F16 ? launch_rows<kF16>(r, tm, grid, s)
+                                       : launch_rows<kBF16>(r, tm, grid, s);
+  }
+  if (wide && src_dtype != INT8KV_F32) {
     a.vecs_per_row = head_dim / 16;
     const int lpt_shift = token_major_shift(num_tokens, num_kv_heads, a.vecs_per_row);
-    const int64_t src_esize = src_dtype == INT8KV_F32 ? 4 : 2;
-    if (lpt_shift >= 0 && static_token_major(num_tokens, num_kv_heads, head_dim, src_esize)) {
+    if (lpt_shift >= 0 && streams) {
       const int lpr_shift = __builtin_ctz((unsigned)a.vecs_per_row);
       const dim3 grid((unsigned)(((num_tokens << lpt_shift) + 255) / 256));
       switch (src_dtype) {
-        case INT8KV_F32:
-          hipLaunchKernelGGL(cache_write16_tm_kernel<kF32>, grid, dim3(256), 0, s, a, lpr_shift, lpt_shift);
-          break;
         case INT8KV_F16:
           hipLaunchKernelGGL(cache_write16_tm_kernel<kF16>, grid, dim3(256), 0, s, a, lpr_shift, lpt_shift);
           break;
@@ -533,9 +723,6 @@ extern "C" int int8kv_cache_write(const void* key, const void* value, int src_dt
     const int64_t blocks16 = (num_tokens * a.vecs_per_row + 255) / 256;
     const dim3 grid((unsigned)blocks16, (unsigned)num_kv_heads);
     switch (src_dtype) {
-      case INT8KV_F32:
-        hipLaunchKernelGGL(cache_write16_kernel<kF32>, grid, dim3(256), 0, s, a);
-        break;
       case INT8KV_F16:
         hipLaunchKernelGGL(cache_write16_kernel<kF16>, grid, dim3(256), 0, s, a);
         break;
@@ -596,23 +783,38 @@ extern "C" int int8kv_dynamic_cache_write(
   hipStream_t s = static_cast<hipStream_t>(stream);
 
   const int32_t vpr16 = head_dim / 16;
-  if (wide_ok(key_cache, value_cache, key_cache_strides, value_cache_strides, num_tokens,
-              num_kv_heads, head_dim) &&
-      (vpr16 & (vpr16 - 1)) == 0) {
+  const bool wide = wide_ok(key_cache, value_cache, key_cache_strides, value_cache_strides,
+                            num_tokens, num_kv_heads, head_dim) &&
+                    (vpr16 & (vpr16 - 1)) == 0;
+  // A slot's kv-head scales as runs of four for 16-byte stores (vec_scales).
+  const bool scales_aligned =
+      k_scale_cache_strides[2] == 1 && v_scale_cache_strides[2] == 1 && num_kv_heads % 4 == 0 &&
+      aligned(k_scale_cache, k_scale_cache_strides[0] * 4, 16) &&
+      aligned(k_scale_cache, k_scale_cache_strides[1] * 4, 16) &&
+      aligned(v_scale_cache, v_scale_cache_strides[0] * 4, 16) &&
+      aligned(v_scale_cache, v_scale_cache_strides[1] * 4, 16);
+  if (wide && use_rows(src_dtype, num_tokens, num_kv_heads, head_dim)) {
+    const int32_t lpr = src_dtype == INT8KV_F32 ? head_dim / 4 : head_dim / 8;
+    if (lpr <= kWave) {
+      DynWriteArgs r = d;
+      r.w.vecs_per_row = lpr;
+      const bool tm = power_of_two(num_kv_heads);
+      r.vec_scales = tm && scales_aligned && 4 * lpr <= kWave;
+      dim3 grid;
+      if (rows_grid(r.w, tm, &grid))
+        return src_dtype == INT8KV_F32   ? launch_dynamic_rows<kF32>(r, tm, grid, s)
+               : src_dtype == INT8KV_F16 ? launch_dynamic_rows<kF16>(r, tm, grid, s)
+                                         : launch_dynamic_rows<kBF16>(r, tm, grid, s);
+    }
+  }
+  if (wide && src_dtype != INT8KV_F32) {
     d.w.vecs_per_row = vpr16;
     const int lpt_shift = token_major_shift(num_tokens, num_kv_heads, vpr16);
     if (lpt_shift >= 0) {
       const int lpr_shift = __builtin_ctz((unsigned)vpr16);
-      d.vec_scales = k_scale_cache_strides[2] == 1 && v_scale_cache_strides[2] == 1 &&
-                     num_kv_heads % 4 == 0 && aligned(k_scale_cache, k_scale_cache_strides[0] * 4, 16) &&
-                     aligned(k_scale_cache, k_scale_cache_strides[1] * 4, 16) &&
-                     aligned(v_scale_cache, v_scale_cache_strides[0] * 4, 16) &&
-                     aligned(v_scale_cache, v_scale_cache_strides[1] * 4, 16);
+      d.vec_scales = scales_aligned;
       const dim3 grid((unsigned)(((num_tokens << lpt_shift) + 255) / 256));
       switch (src_dtype) {
-        case INT8KV_F32:
-          hipLaunchKernelGGL(dynamic_write16_tm_kernel<kF32>, grid, dim3(256), 0, s, d, lpr_shift, lpt_shift);
-          break;
         case INT8KV_F16:
           hipLaunchKernelGGL(dynamic_write16_tm_kernel<kF16>, grid, dim3(256), 0, s, d, lpr_shift, lpt_shift);
           break;
@@ -625,9 +827,6 @@ extern "C" int int8kv_dynamic_cache_write(
     const int64_t blocks16 = (num_tokens * vpr16 + 255) / 256;
     const dim3 grid((unsigned)blocks16, (unsigned)num_kv_heads);
     switch (src_dtype) {
-      case INT8KV_F32:
-        hipLaunchKernelGGL(dynamic_write16_kernel<kF32>, grid, dim3(256), 0, s, d);
-        break;
       case INT8KV_F16:
         hipLaunchKernelGGL(dynamic_write16_kernel<kF16>, grid, dim3(256), 0, s, d);
         break;

@@ -1,0 +1,66 @@
+"""Cache writes on both sides of the row kernels' bounds (one 16-byte load per lane: fp32 sources at
+every size, 16-bit ones below 2^20 elements), bit-exact against the oracle."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import int8kv
+from int8kv import cache_ops
+from oracle import int8kv_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# (tokens, kv heads, head_dim): one token; rows of 10 pieces; kv heads no power of two; more lanes
+# per token than a wave; 2^20 elements and one token fewer; fp32 past the Infinity Cache (256 MB).
+SHAPES = [(1, 4, 128), (37, 2, 80), (130, 3, 64), (63, 8, 256), (2047, 4, 128), (2048, 4, 128)]
+LARGE = [(60000, 4, 128)]
+
+
+def _inputs(tokens, hkv, d, dtype, dev, seed):
+    g = torch.Generator().manual_seed(seed)
+    k = (torch.randn(tokens, hkv, d, generator=g) * 3).to(dtype)
+    v = torch.randn(tokens, hkv, d, generator=g).to(dtype)
+    blocks = tokens // 16 + 2
+    slots = torch.randperm(blocks * 16, generator=g)[:tokens]
+    slots[::7] = -1
+    if tokens > 2:
+        slots[1] = blocks * 16 + 5  # past the cache
+    return k, v, slots, torch.zeros(blocks, 16, hkv, d, dtype=torch.int8)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,hkv,d", SHAPES + LARGE)
+def test_static_write(cuda, tokens, hkv, d, dtype):
+    if tokens >= 60000 and dtype != torch.float32:
+        pytest.skip("16-bit sources of this size take the kernels tested elsewhere")
+    k, v, slots, cache = _inputs(tokens, hkv, d, dtype, cuda, tokens + d)
+    ks = torch.linspace(0.01, 0.08, hkv)
+    vs = torch.linspace(0.03, 0.005, hkv)
+    kc, vc = cache.to(cuda), cache.to(cuda)
+    int8kv.int8_kv_cache_write(k.to(cuda), v.to(cuda), kc, vc, slots.to(cuda), ks.to(cuda), vs.to(cuda))
+    rk, rv = cache.numpy().copy(), cache.numpy().copy()
+    keep = (slots >= 0) & (slots < cache.shape[0] * 16)
+    O.int8_kv_cache_write(k[keep].float().numpy(), v[keep].float().numpy(), rk, rv,
+                          slots[keep].numpy(), ks.numpy(), vs.numpy())
+    assert np.array_equal(kc.cpu().numpy(), rk) and np.array_equal(vc.cpu().numpy(), rv)
+
+
+@pytest.mark.parametrize("strided_scales", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tokens,hkv,d", [s for s in SHAPES if s[2] != 80] + [(40, 4, 512), (40, 4, 256)])
+def test_dynamic_write(cuda, tokens, hkv, d, dtype, strided_scales):
+    k, v, slots, cache = _inputs(tokens, hkv, d, dtype, cuda, 3 * tokens + d)
+    kc, vc = cache.to(cuda), cache.to(cuda)
+    step = 2 if strided_scales else 1
+    ksc, vsc = (torch.zeros(cache.shape[0], 16, hkv * step, device=cuda)[..., ::step] for _ in range(2))
+    cache_ops.reshape_and_cache_int8(k.to(cuda), v.to(cuda), kc, vc, ksc, vsc, slots.to(cuda))
+    rk, rv = cache.numpy().copy(), cache.numpy().copy()
+    rks, rvs = (np.zeros((cache.shape[0], 16, hkv), np.float32) for _ in range(2))
+    keep = (slots >= 0) & (slots < cache.shape[0] * 16)
+    O.reshape_and_cache_int8(k[keep].float().numpy(), v[keep].float().numpy(), rk, rv, rks, rvs,
+                             slots[keep].numpy())
+    assert np.array_equal(kc.cpu().numpy(), rk) and np.array_equal(vc.cpu().numpy(), rv)
+    assert np.array_equal(ksc.cpu().numpy(), rks) and np.array_equal(vsc.cpu().numpy(), rvs)
