@@ -216,12 +216,13 @@ __global__ __launch_bounds__(kWaves * 64) void skinny_kernel(LinearArgs a) {
         const f32x4 ulo = column_sum(2);
         const f32x4 uhi = column_sum(3);
         const float u[8] = {ulo[0], ulo[1], ulo[2], ulo[3], uhi[0], uhi[1], uhi[2], uhi[3]};
-        float g[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) g[j] = round_bf16(y[j]);
-        silu(g, y);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) y[j] = round_bf16(y[j]) * round_bf16(u[j]);
+        for (int j = 0; j < 8; ++j) {
+          const float g = round_bf16(y[j]);
+          const float mid = silu_middle(g);
+          const float end = silu_ends(g);  // (no branch: its values would need registers x and W hold)
+          y[j] = round_bf16(fabsf(g) < kSiluMiddle ? mid : end) * round_bf16(u[j]);
+        }
       }
       const int64_t col = kRowsPerTile * (int64_t)tile + 8 * h;
       if constexpr (EPI == kEpiPart) {

@@ -97,3 +97,30 @@ def test_step_falls_back_to_torch_products(cuda, batch, hidden):
     loop.prefill(torch.zeros(batch, 5, dtype=torch.int64))
     loop.step_eager()
     assert torch.isfinite(loop.logits.float()).all()
+
+
+def test_silu_of_every_bf16_value(cuda):
+    """All 65536 gate values (both branches of silu.h, infinities, NaN, denormals) and the fused
+    product's copy of it: within half a bf16 spacing, with 2^-10 of one for the fp32 error, of the
+    float64 value; -0 where exp(-g) overflows fp32; a NaN stays one."""
+    bits = torch.arange(1 << 16, dtype=torch.int32)
+    gate = (bits << 16).view(torch.float32).to(torch.bfloat16).view(32, 2048)
+    ref = gate.double() / (1 + torch.exp(-gate.double()))
+    ref = torch.where(gate == float("-inf"), torch.zeros_like(ref), ref)
+    ref = torch.where(gate.double() < -88.7228394, torch.zeros_like(ref), ref)
+    gate_up = torch.cat([gate, torch.ones_like(gate)], dim=1).to(cuda)
+    out = DL.hip_silu_mul(gate_up, torch.empty(32, 2048, dtype=torch.bfloat16, device=cuda)).cpu().double()
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    fine = torch.isfinite(ref)
+    assert torch.equal(out[torch.isinf(ref)], ref[torch.isinf(ref)])
+    spacing = torch.exp2(torch.floor(torch.log2(ref[fine].abs().clamp_min(2.0**-126))) - 7)
+    assert ((out[fine] - ref[fine]).abs() <= spacing * (0.5 + 2.0**-10)).all()
+    # The fused product with w = identity rows gives the same bits.
+    x = torch.zeros(32, 64, dtype=torch.bfloat16, device=cuda)
+    x[:, :16] = torch.randn(32, 16, device=cuda).to(torch.bfloat16) * 120
+    w = torch.zeros(32, 64, dtype=torch.bfloat16, device=cuda)
+    w[:16, :16] = torch.eye(16, device=cuda)
+    w[16:, 0] = 1
+    fused = DL.hip_linear_silu_mul(x, w, torch.empty(32, 16, dtype=torch.bfloat16, device=cuda))
+    gu = torch.cat([x[:, :16], x[:, :1].expand(32, 16)], dim=1).contiguous()
+    assert torch.equal(fused, DL.hip_silu_mul(gu, torch.empty_like(fused)))
