@@ -546,7 +546,11 @@ int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_hea
   // at head_dim 256 it measured 1 % slower (659 -> 666 us), and padded head_dims and kv-head
   // pairs (k_run order) are not measured with it.  The per-sequence kernels read without it.
   const int64_t touch_blocks = batch * table_width < num_blocks ? batch * table_width : num_blocks;
-  p.nt = (i8 || (hd == 128 && !p.pad && !p.kv_pair)) && !p.group_mode &&
+  // Padded INT8 rows are no whole lines: the hint had the waves of neighbouring heads fetch the
+  // lines they share again (HIP-graph replays, us with / without it: 32 x 96 heads, 40 x U[1, 4000]
+  // 139 / 102; 32 x 80, 4 x 30000 224 / 144; 8 x 96, 32 x 8000 116 / 89; 8 x 160, 32 x 6000 163 /
+  // 111; 8 x 48, 64 x 8000 113 / 103).
+  p.nt = (i8 || (hd == 128 && !p.kv_pair)) && !p.pad && !p.group_mode &&
          (double)touch_blocks * block_size * num_kv_heads * head_dim * ce * 2 >
              (double)kNonTemporalMinBytes;
   *hp = p;

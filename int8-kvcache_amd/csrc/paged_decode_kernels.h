@@ -1871,13 +1871,19 @@ inline void launch_main(const DecodeArgs& a, dim3 grid, int W, hipStream_t s) {
 template <int CACHE, int QT, int HD, bool PAIR, bool PAD>
 void launch_ranges(const DecodeArgs& a, dim3 grid, int W, bool nt, hipStream_t s) {
   constexpr int KH = PAIR ? 128 : HD;
-  // INT8 caches: non-temporal loads for large pools, int8 scores for a quantised query.
+  // INT8 caches: non-temporal loads for large pools (whole-line rows: plan_call decides), int8
+  // scores for a quantised query.
   if constexpr (CACHE == kI8) {
-    if (nt && a.quantize_q)
-      launch_main<CACHE, QT, true, true, KH, PAIR, PAD>(a, grid, W, s);
-    else if (nt)
-      launch_main<CACHE, QT, true, false, KH, PAIR, PAD>(a, grid, W, s);
-    else if (a.quantize_q)
+    if constexpr (!PAD) {
+      if (nt) {
+        if (a.quantize_q)
+          launch_main<CACHE, QT, true, true, KH, PAIR, PAD>(a, grid, W, s);
+        else
+          launch_main<CACHE, QT, true, false, KH, PAIR, PAD>(a, grid, W, s);
+        return;
+      }
+    }
+    if (a.quantize_q)
       launch_main<CACHE, QT, false, true, KH, PAIR, PAD>(a, grid, W, s);
     else
       launch_main<CACHE, QT, false, false, KH, PAIR, PAD>(a, grid, W, s);
