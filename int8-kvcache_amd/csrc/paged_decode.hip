@@ -513,6 +513,12 @@ int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_hea
   if (p.ct > 0) p.seq_cost = kSeqStartCostWide;
   // Four tiles in flight leave no registers for an fp32 query's lo operands: two for those.
   p.launch_depth = p.group_mode ? 2 : (p.depth == 4 && query_dtype != INT8KV_F32 ? 4 : 2);
+  // Per-sequence workgroups whose waves can hold one tile at most request one (group_kernel; the
+  // padded instances keep two).
+  if (p.group_mode && !pad) {
+    const int64_t waves = (int64_t)(hd > 128 ? group_waves<256>() : group_waves<128>()) * std::max(p.split, 1);
+    if (std::ceil((double)table_width * block_size / tile_tokens) <= (double)waves) p.launch_depth = 1;
+  }
   // Units of one sequence are at most ceil(table_width x block_size / 32) + seq_cost (lengths are
   // clamped to the table); 64 of them fit the 32-bit wave scans unless one sequence could hold
   // more than 2^25 tiles.

@@ -1429,7 +1429,14 @@ __device__ __forceinline__ bool share_may_hold(int v, int smax, int nw) {
   return false;
 }
 
-template <int CACHE, int QT, bool QQ, int HD, bool SPLIT, bool PAD = false>
+// DEPTH: 2 tiles in flight per wave, or 1 where no wave can hold more than one tile (plan_call): a
+// wave's second request would read its only tile again, and with eight waves on one compute unit
+// those requests are what the first tiles wait for (a unit takes K loads, four rows to a quad of
+// lanes, at 16 and V loads at 17.7 bytes per clock).  us per call, HIP-graph replays, 2 -> 1: 28 / 4
+// heads, INT8: 1 x 256 7.41 -> 6.09, 64 x 250 8.50 -> 7.27, split 1 x 2048 9.31 -> 8.80, 8 x 1024
+// 9.52 -> 8.85; BF16 1 x 256 8.78 -> 6.53, 8 x 1024 10.76 -> 9.58; head_dim 256 INT8 1 x 128 8.66
+// -> 7.50.
+template <int CACHE, int QT, bool QQ, int HD, bool SPLIT, bool PAD = false, int DEPTH = 2>
 __global__ __launch_bounds__(group_waves<HD>() * 64) __attribute__((amdgpu_waves_per_eu(HD > 128 ? 1 : 2))) void group_kernel(DecodeArgs a) {
   constexpr int NW = group_waves<HD>();
   __shared__ int32_t s_ids[NW][kChunkTiles * tile_blocks<CACHE>()];
@@ -1496,7 +1503,7 @@ __global__ __launch_bounds__(group_waves<HD>() * 64) __attribute__((amdgpu_waves
     // still precedes the block-id loads, which is all run_segment's waits assume.)
     if (!SPLIT && !early_q)
       issue_query<QT, HD, false, PAD, CACHE != kI8>(a, b, hm, li, lg, qraw);
-    run_segment<CACHE, QT, false, QQ, HD, 2, true, false, PAD, !SPLIT>(
+    run_segment<CACHE, QT, false, QQ, HD, DEPTH, true, false, PAD, !SPLIT>(
         a, s_ids[wave], b, L, vh, ta, tb, false, 0, lane, s_acc[wave], s_m[wave], s_l[wave],
         &qraw INT8KV_STAMPS_ARG);
   } else if (li < G) {  // no tiles for this wave: the neutral state
@@ -1965,17 +1972,27 @@ int launch(const DecodeArgs& a, const HostPlan& hp, uint32_t flags, hipStream_t 
     if (flags & INT8KV_DECODE_MAIN) {
       dim3 grid((unsigned)a.batch, (unsigned)a.num_kv_heads, (unsigned)(a.split > 0 ? a.split : 1));
       const dim3 block(group_waves<HD>() * kWave);
-      if (a.split > 0) {
-        if (a.quantize_q)
-          hipLaunchKernelGGL((group_kernel<CACHE, QT, true, HD, true, PAD>), grid, block, 0, s, a);
+      auto group = [&](auto depth) {
+        constexpr int D = decltype(depth)::value;
+        if (a.split > 0) {
+          if (a.quantize_q)
+            hipLaunchKernelGGL((group_kernel<CACHE, QT, true, HD, true, PAD, D>), grid, block, 0, s, a);
+          else
+            hipLaunchKernelGGL((group_kernel<CACHE, QT, false, HD, true, PAD, D>), grid, block, 0, s, a);
+        } else {
+          if (a.quantize_q)
+            hipLaunchKernelGGL((group_kernel<CACHE, QT, true, HD, false, PAD, D>), grid, block, 0, s, a);
+          else
+            hipLaunchKernelGGL((group_kernel<CACHE, QT, false, HD, false, PAD, D>), grid, block, 0, s, a);
+        }
+      };
+      if constexpr (!PAD) {
+        if (hp.launch_depth == 1)
+          group(std::integral_constant<int, 1>{});
         else
-          hipLaunchKernelGGL((group_kernel<CACHE, QT, false, HD, true, PAD>), grid, block, 0, s, a);
+          group(std::integral_constant<int, 2>{});
       } else {
-        if (a.quantize_q)
-          hipLaunchKernelGGL((group_kernel<CACHE, QT, true, HD, false, PAD>), grid, block, 0, s, a);
-        else
-          hipLaunchKernelGGL((group_kernel<CACHE, QT, false, HD, false, PAD>), grid, block, 0, s,
-                             a);
+        group(std::integral_constant<int, 2>{});
       }
       hipError_t e = hipGetLastError();
       if (e != hipSuccess) return (int)e;

@@ -244,3 +244,30 @@ def test_groups_above_16_several_tiles_per_wave(cuda, hq, hkv, d, cache):
     out = int8kv.bf16_paged_attention(q, k_cpu.to(cuda), v_cpu.to(cuda), bt, sl)
     assert (out[0] == 0).all() and (out[10] == 0).all()
     _check(out, ref, f"{hq}/{hkv} d={d} {cache}")
+
+
+@pytest.mark.parametrize("cache", ["int8", "bf16"])
+@pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (28, 4, 128), (16, 8, 256)])
+def test_one_tile_per_wave_bound(cuda, hq, hkv, d, cache):
+    """Per-sequence workgroups at the bound of one tile per wave (8 waves, 4 at head_dim 256) and one
+    block past it, single-pass and split: the instance with one tile in flight and the one with
+    two, on sequences of no, one, some and all tiles."""
+    waves = 8 if d <= 128 else 4
+    for splits in (1, 4):
+        most = splits * waves * 32
+        for longest in (most, most + 16):
+            lens = [longest, 0, 1, 31, 33, most // 2 + 5, most - 1, longest - 16]
+            c = decode_case(lens, seed=longest + d, hq=hq, hkv=hkv, head_dim=d, extra_blocks=3)
+            q, kc, vc, bt, sl, ks, vs = to_dev(c, cuda)
+            if cache == "int8":
+                ref = oracle_int8(c)
+                out = int8kv.int8_paged_attention(q, kc, vc, bt, sl, ks, vs, num_splits=splits)
+            else:
+                k_cpu, v_cpu = bf16_caches(c)
+                ref = O.paged_attention_ref(c.query.float().numpy(), k_cpu.float().numpy(),
+                                            v_cpu.float().numpy(), c.block_tables.numpy(),
+                                            c.seq_lens.numpy())
+                out = int8kv.bf16_paged_attention(q, k_cpu.to(cuda), v_cpu.to(cuda), bt, sl,
+                                                  num_splits=splits)
+            assert (out[1] == 0).all()
+            _check(out, ref, f"{cache} d={d} splits={splits} longest={longest}")
