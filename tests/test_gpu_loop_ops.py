@@ -199,3 +199,31 @@ def test_argmax_rows_matches_torch(cuda):
     assert torch.equal(out3, short.argmax(-1))
     assert out[1].item() == 1000 and out[6].item() == 0 and out[4].item() == 5
     assert out3[7].item() == 152_058 and out3[8].item() == 3 and out[9].item() == 20
+
+
+@pytest.mark.parametrize("vocab", [5, 8, 13, 8 * 1024, 8 * 8 * 1024 + 8, 152064])
+def test_argmax_rows_orders_special_values(cuda, vocab):
+    """Rows that the comparison of whole vectors could get wrong: signed zeros and equal maxima in
+    different vectors, all -inf, all negative, +inf, and NaN of either sign; one row per kind."""
+    inf, nan = float("inf"), float("nan")
+    g = torch.Generator().manual_seed(vocab)
+    base = -torch.rand(8, vocab, generator=g) - 0.5
+    first, last = vocab // 3, vocab - 1
+    want = base.to(torch.bfloat16).float().argmax(-1)
+    for row, (a, b) in enumerate([(-0.0, 0.0), (0.0, -0.0), (3.0, 3.0), (inf, inf)]):
+        base[row, first], base[row, last] = a, b
+        want[row] = first
+    base[4] = -inf
+    want[4] = 0
+    base[5, last] = nan
+    want[5] = last
+    x = base.to(torch.bfloat16)
+    want[7] = x[7].float().argmax()
+    bits = x.view(torch.int16)
+    bits[6, first] = -1  # a NaN with the sign set, before a larger ordinary value
+    x[6, last] = inf if last != first else x[6, last]
+    want[6] = first
+    want[7] = int((x[7] == x[7].max()).nonzero()[0])
+    out = torch.empty(8, dtype=torch.int64, device=cuda)
+    DL.hip_argmax_rows(x.to(cuda), out)
+    assert out.tolist() == want.tolist()
