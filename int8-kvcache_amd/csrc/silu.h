@@ -29,13 +29,14 @@ __device__ __forceinline__ float silu_middle(float g) {
 }
 
 // The rest: g itself above (1 + exp(-g) is 1 there), g exp(g) below, with exp(g) 2^64 in range
-// (1 + exp(-g) is exp(-g) there), and -0 from where exp(-g) overflows fp32.  A NaN stays one.
+// (1 + exp(-g) is exp(-g) there), and -0 from where exp(-g) overflows fp32, as g / infinity.  -inf
+// gives NaN there too (-inf / inf, as torch's silu), and a NaN stays one.
 __device__ __forceinline__ float silu_ends(float g) {
   const float t = g * kLog2eHi;
   const float lo = fmaf(g, kLog2eHi, -t) + g * kLog2eLo;
   const float x = __builtin_amdgcn_exp2f(t + 64.0f);
   const float low = g * fmaf(x * kLn2, lo, x) * 0x1p-64f;
-  return g > 0.0f ? g : (g < -88.7228394f ? -0.0f : low);
+  return g > 0.0f ? g : (g < -88.7228394f ? g * 0.0f : low);
 }
 
 __device__ __forceinline__ float silu(float g) {

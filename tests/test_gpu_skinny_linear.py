@@ -102,12 +102,14 @@ def test_step_falls_back_to_torch_products(cuda, batch, hidden):
 def test_silu_of_every_bf16_value(cuda):
     """All 65536 gate values (both branches of silu.h, infinities, NaN, denormals) and the fused
     product's copy of it: within half a bf16 spacing, with 2^-10 of one for the fp32 error, of the
-    float64 value; -0 where exp(-g) overflows fp32; a NaN stays one."""
+    float64 value; -0 where exp(-g) overflows fp32; a NaN stays one and -inf becomes one, as in
+    torch.nn.functional.silu."""
     bits = torch.arange(1 << 16, dtype=torch.int32)
     gate = (bits << 16).view(torch.float32).to(torch.bfloat16).view(32, 2048)
     ref = gate.double() / (1 + torch.exp(-gate.double()))
-    ref = torch.where(gate == float("-inf"), torch.zeros_like(ref), ref)
-    ref = torch.where(gate.double() < -88.7228394, torch.zeros_like(ref), ref)
+    overflows = (gate.double() < -88.7228394) & torch.isfinite(gate)
+    ref = torch.where(overflows, torch.zeros_like(ref), ref)
+    assert torch.equal(torch.isnan(ref), torch.isnan(torch.nn.functional.silu(gate.double())))
     gate_up = torch.cat([gate, torch.ones_like(gate)], dim=1).to(cuda)
     out = DL.hip_silu_mul(gate_up, torch.empty(32, 2048, dtype=torch.bfloat16, device=cuda)).cpu().double()
     assert torch.equal(torch.isnan(out), torch.isnan(ref))
@@ -115,12 +117,20 @@ def test_silu_of_every_bf16_value(cuda):
     assert torch.equal(out[torch.isinf(ref)], ref[torch.isinf(ref)])
     spacing = torch.exp2(torch.floor(torch.log2(ref[fine].abs().clamp_min(2.0**-126))) - 7)
     assert ((out[fine] - ref[fine]).abs() <= spacing * (0.5 + 2.0**-10)).all()
-    # The fused product with w = identity rows gives the same bits.
+    # The fused product with w = a diagonal gives the same values (column 5 overflows to -inf in
+    # row 3 and +inf in row 4: inputs of -inf itself would put 0 x inf into the other columns).
     x = torch.zeros(32, 64, dtype=torch.bfloat16, device=cuda)
     x[:, :16] = torch.randn(32, 16, device=cuda).to(torch.bfloat16) * 120
+    x[3, 5], x[4, 5] = -3e38, 3e38
+    diag = torch.ones(16, device=cuda)
+    diag[5] = 2.0**40
     w = torch.zeros(32, 64, dtype=torch.bfloat16, device=cuda)
-    w[:16, :16] = torch.eye(16, device=cuda)
+    w[:16, :16] = torch.diag(diag)
     w[16:, 0] = 1
     fused = DL.hip_linear_silu_mul(x, w, torch.empty(32, 16, dtype=torch.bfloat16, device=cuda))
-    gu = torch.cat([x[:, :16], x[:, :1].expand(32, 16)], dim=1).contiguous()
-    assert torch.equal(fused, DL.hip_silu_mul(gu, torch.empty_like(fused)))
+    gate = (x[:, :16].float() * diag).to(torch.bfloat16)
+    gu = torch.cat([gate, x[:, :1].expand(32, 16)], dim=1).contiguous()
+    ref = DL.hip_silu_mul(gu, torch.empty_like(fused))
+    assert torch.isnan(ref[3, 5]) and torch.isinf(ref[4, 5]) and torch.isnan(ref).sum() == 1
+    assert torch.equal(torch.isnan(fused), torch.isnan(ref))
+    assert torch.equal(torch.nan_to_num(fused), torch.nan_to_num(ref))
