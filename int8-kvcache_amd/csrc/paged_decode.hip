@@ -494,14 +494,16 @@ int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_hea
     for (int32_t waves = (tiles + most - 1) / most; waves < tiles; ++waves) {
       const int32_t heads = num_kv_heads * waves;  // workgroups per range
       if (units * heads < (double)kWideMinUnits * cus) continue;
+      // ct tiles a wave may need fewer waves than were counted (5 tiles on 4 waves: 2 + 2 + 1):
+      // a workgroup without query heads would read the whole cache for nothing.
       p.ct = (tiles + waves - 1) / waves;
-      p.col_tiles = waves;
-      p.grid_heads = heads;
+      p.col_tiles = (tiles + p.ct - 1) / p.ct;
+      p.grid_heads = num_kv_heads * p.col_tiles;
       p.depth = 2;
       p.halves = 1;
       p.pair_min = 0x7fffffff;
       if (auto_ranges_req)
-        p.launch_ranges = (int32_t)std::max<int64_t>(1, std::min<int64_t>(num_ranges, cus / heads));
+        p.launch_ranges = (int32_t)std::max<int64_t>(1, std::min<int64_t>(num_ranges, cus / p.grid_heads));
       if (automatic) p.launch_min_tiles = std::max(min_tiles, kWideMinUnits);
       break;
     }
@@ -727,6 +729,27 @@ extern "C" int int8kv_decode_plan(int query_dtype, int cache_dtype, int64_t batc
   p.compute_units = (int32_t)cus;
   p.workspace_bytes = hp.need;
   *plan = p;
+  return INT8KV_OK;
+}
+
+// How the range layout's launch spreads groups above 16 query heads, for the planner's tests (not
+// part of the public C ABI).  columns: column tiles of 16 query heads per wave (0: one wave per
+// tile), grid heads, ranges and smallest range launched.
+extern "C" int int8kv_decode_plan_columns(int query_dtype, int cache_dtype, int64_t batch,
+                                          int32_t num_q_heads, int32_t num_kv_heads,
+                                          int32_t head_dim, int64_t num_blocks, int32_t block_size,
+                                          int64_t table_width, int32_t num_ranges,
+                                          int32_t min_tiles, uint32_t flags, int32_t compute_units,
+                                          int32_t columns[4]) {
+  HostPlan hp;
+  const int st = plan_call(query_dtype, cache_dtype, batch, num_q_heads, num_kv_heads, head_dim,
+                           num_blocks, block_size, table_width, head_dim, head_dim, num_ranges,
+                           min_tiles, flags, compute_units, 0, &hp);
+  if (st != INT8KV_OK) return st;
+  columns[0] = hp.ct;
+  columns[1] = hp.grid_heads;
+  columns[2] = hp.launch_ranges;
+  columns[3] = hp.launch_min_tiles;
   return INT8KV_OK;
 }
 

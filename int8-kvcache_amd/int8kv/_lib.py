@@ -104,6 +104,12 @@ def bind(path: Path) -> ctypes.CDLL:
         ctypes.c_int, ctypes.c_int, i64, i32, i32, i32, i64, i32, i64, i64, i64, i32, i32, u32, i32,
         i32, ctypes.POINTER(DecodePlan),
     ]
+    # csrc/paged_decode.hip (for the planner's tests, not part of the public C ABI)
+    lib.int8kv_decode_plan_columns.restype = ctypes.c_int
+    lib.int8kv_decode_plan_columns.argtypes = [
+        ctypes.c_int, ctypes.c_int, i64, i32, i32, i32, i64, i32, i64, i32, i32, u32, i32,
+        ctypes.POINTER(i32),
+    ]
     lib.int8kv_paged_decode.restype = ctypes.c_int
     lib.int8kv_paged_decode.argtypes = [
         _vp, ctypes.c_int, i64, i32, i32, _c_i64p, _vp, _vp, ctypes.c_int, i64, i32, i32,

@@ -11,6 +11,8 @@ two functions' outputs for given sizes.
 
 from __future__ import annotations
 
+import ctypes
+
 import pytest
 import torch
 
@@ -347,6 +349,34 @@ def test_groups_above_16_take_column_tiles():
     # MQA with 64 query heads: 4 grid heads, the automatic count of 4 kv heads
     assert plan(hq=64, hkv=1, batch=64, width=2048)["num_ranges"] == \
         plan(hq=28, hkv=4, batch=64, width=2048)["num_ranges"]
+
+
+def _columns(cache=I8, batch=1, hq=64, hkv=1, d=64, width=32, cus=256, bs=16, query=Q, ranges=0,
+             min_tiles=0, flags=_lib.DECODE_ALL):
+    """(column tiles per wave, grid heads, ranges, smallest range) of the range layout's launch."""
+    out = (ctypes.c_int32 * 4)()
+    _lib.check(_lib.load().int8kv_decode_plan_columns(
+        _lib.DTYPE_CODE[query], _lib.DTYPE_CODE[cache], batch, hq, hkv, d, batch * width + 16, bs,
+        width, ranges, min_tiles, flags, cus, out), "int8kv_decode_plan_columns")
+    return tuple(out)
+
+
+def test_groups_above_16_leave_no_grid_head_empty():
+    """However the column tiles are spread over waves, every wave has a tile and every tile a wave."""
+    spread = set()
+    for cache in (I8, BF16):
+        for d in (48, 64, 96, 128, 256):
+            for hkv in (1, 2, 3):
+                for group in (17, 33, 48, 49, 64, 71, 96, 100, 128, 160, 192, 256):
+                    tiles = -(-group // 16)
+                    for batch, width in ((2, 1024), (5, 384), (7, 160), (9, 160), (6, 160), (4, 256),
+                                         (40, 256), (16, 64), (200, 32), (300, 9)):
+                        ct, heads, ranges, _ = _columns(cache, batch, group * hkv, hkv, d, width)
+                        waves, rest = divmod(heads, hkv)
+                        assert rest == 0 and ranges >= 1
+                        assert waves == -(-tiles // max(ct, 1)), (group, hkv, d, batch, width, ct, heads)
+                        spread.add((tiles, ct))
+    assert {(5, 2), (5, 3), (6, 2), (4, 2)} <= spread
 
 
 def test_plan_rejects_what_the_decode_rejects():

@@ -246,6 +246,29 @@ def test_groups_above_16_several_tiles_per_wave(cuda, hq, hkv, d, cache):
     _check(out, ref, f"{hq}/{hkv} d={d} {cache}")
 
 
+# Calls of less work, whose column tiles are spread over more waves than registers would need: 5 as
+# 3 + 2 and 2 + 2 + 1, 6 as 2 + 2 + 2, 4 as 2 + 2 (query heads, kv heads, head_dim, batch, tokens).
+@pytest.mark.parametrize("cache", ["int8", "bf16"])
+@pytest.mark.parametrize("hq,hkv,d,batch,tokens", [
+    (71, 1, 64, 2, 16384), (71, 1, 64, 5, 6144), (71, 1, 64, 7, 2560), (71, 1, 128, 7, 2560),
+    (96, 1, 64, 6, 2560), (64, 1, 64, 9, 2560), (34, 2, 128, 9, 2560)])
+def test_groups_above_16_spread_over_waves(cuda, hq, hkv, d, batch, tokens, cache):
+    lens = [tokens] + [tokens - 37 * i for i in range(1, batch)]
+    c = decode_case(lens, seed=hq + batch, hq=hq, hkv=hkv, head_dim=d, extra_blocks=5)
+    q, kc, vc, bt, sl, ks, vs = to_dev(c, cuda)
+    if cache == "int8":
+        full, out = _decode_auto(q, kc, vc, bt, sl, ks, vs)
+        _untouched(full, d, f"{hq}/{hkv} d={d} {batch}x{tokens}")
+        ref = oracle_int8(c)
+    else:
+        k_cpu, v_cpu = bf16_caches(c)
+        ref = O.paged_attention_ref(c.query.float().numpy(), k_cpu.float().numpy(),
+                                    v_cpu.float().numpy(), c.block_tables.numpy(),
+                                    c.seq_lens.numpy())
+        out = int8kv.bf16_paged_attention(q, k_cpu.to(cuda), v_cpu.to(cuda), bt, sl)
+    _check(out, ref, f"{cache} {hq}/{hkv} d={d} {batch}x{tokens}")
+
+
 @pytest.mark.parametrize("cache", ["int8", "bf16"])
 @pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (28, 4, 128), (16, 8, 256)])
 def test_one_tile_per_wave_bound(cuda, hq, hkv, d, cache):
