@@ -86,6 +86,7 @@ constexpr int kSeqStartCostWide = 14;
 constexpr int kMinTilesSmall = 2;
 constexpr int kMinTilesLarge = 4;
 constexpr int kWideMinUnits = 8;  // groups above 16: two tiles for each of a workgroup's four waves
+constexpr int kWideLeastUnits = 5;  // units a workgroup below which one wave per column tile is used
 constexpr int64_t kMaxMergeRanges = 128;  // ranges per sequence the merge takes in 4 rounds
 // Resident decode waves per CU the automatic range count targets: one per SIMD.  Against two
 // per SIMD (the second of which streams ~30 % slower) it measured 3-11 % faster on every
@@ -273,6 +274,61 @@ int32_t auto_ranges_for(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_
   const int32_t most = wide_most_tiles(padded_head_dim(head_dim));
   if (tiles == 1 || most == 1) return r;
   return std::max(r, (int32_t)(cu / (num_kv_heads * ((tiles + most - 1) / most))));
+}
+
+// Column tiles per wave of the wide kernel (paged_decode_wide.h) for a range-layout call with
+// `tiles` column tiles per kv head, or 0 for one wave per tile (decode_kernel).  seq_tiles: 32-token
+// tiles of the longest possible sequence; per_cu: units of one kv head set per compute unit.
+// Measured on MI355X over 734 calls (2-8 tiles, head_dim 64 and 128, 32 to 51,200 tokens per kv
+// head, uniform and ragged, INT8 and BF16 caches), us one wave per tile -> wide:
+//   * Two tiles per wave win from about 5 units a workgroup on, since each halves the K/V operands built
+//     (71/1 heads x 64, 7 x 2560: 16.6 -> 13.6; 96/1 x 128, 10 x 4096: 27.3 -> 21.5).  More tiles
+//     per wave cost more per range (states, records: ~10 us at 2, ~12 at 3, ~18 at 5 on one
+//     workgroup) and less per unit, so each count has its own least per_cu, larger where one
+//     workgroup holds all tiles (71/1 x 64, 16 / 24 / 40 x 4096 with 2, 3, 5 tiles: 18.5 18.3
+//     21.2 / 23.1 21.3 23.7 / 30.6 28.1 26.6), and must save a tenth of the arithmetic (~3 + 2 ct per
+//     wave and unit): 8 tiles as 3 + 3 + 2 never beat 4 x 2.
+//   * decode_kernel's workgroup of four waves on one kv head shares its lines in L1 and gains
+//     less.  Against it the wide kernel's costlier sequence starts lose below 32 tiles a
+//     sequence (64/1 x 64, 400 x 512: 40.7 -> 41.4; below 16 tiles always: 300 x 130 23.2 ->
+//     27.4), and at head_dim 128 with two tiles per kv head below 48 tiles and 40 units (40/2 x
+//     128, 100 x 1000: 27.9 -> 30.0, BF16 16 x 4096 21.9 -> 23.7; 64 x 4096 48.0 -> 39.1).
+//   * A quantised query's int8 score products have no wide form.  At head_dim 128 four
+//     sharing waves are then the faster ones up to 32 units (64/1 x 128, 40 x 4096: 32.4 against
+//     33.6 wide; 8 x 32768 42.5 -> 38.5), 64 with two tiles; others up to 6 (71/1, 10 x 4096 20.9
+//     against 22.1).
+//   * 16-bit caches at 128 with three workgroups per range (ranges no multiple of the 8 XCDs, so
+//     that the three read the range's lines through different L2s): slower from 9 x 2560 on
+//     (71/1 x 128, 40 x 4096 41.4 -> 48.9).
+int32_t wide_column_tiles(bool int8_cache, bool quantised, int32_t hd, int32_t tiles,
+                          int32_t num_kv_heads, double seq_tiles, double per_cu) {
+  const int32_t most = wide_most_tiles(hd);
+  if (tiles < 2 || most < 2) return 0;
+  const bool shared = waves_per_wg(num_kv_heads * tiles) == 4;
+  const double shortest = !shared ? (int8_cache || hd == 64 ? 16 : 32)
+                                  : (hd == 128 && tiles == 2 ? 48 : 32);
+  if (seq_tiles < shortest) return 0;
+  if (hd == 128) {
+    const double least = !shared     ? (quantised ? 6 : 0)
+                         : tiles > 2 ? (quantised ? 32 : 0)
+                                     : (quantised ? 64 : 40);
+    if (per_cu < least) return 0;
+  }
+  const auto cost = [](int32_t waves, int32_t ct) { return waves * (3 + 2 * ct); };
+  int32_t ct = 2;
+  int32_t waves = (tiles + 1) / 2;
+  if (per_cu * waves < kWideLeastUnits) return 0;
+  for (int32_t w = waves - 1; w >= (tiles + most - 1) / most; --w) {
+    const int32_t c = (tiles + w - 1) / w;
+    if ((tiles + c - 1) / c < w) continue;  // (c tiles a wave need fewer waves)
+    const double least = w > 1 ? (c == 3 ? 8 : 12) : (c == 3 ? 12 : c == 4 ? 30 : 18);
+    if (per_cu >= least && 10 * cost(w, c) <= 9 * cost(waves, ct)) {
+      ct = c;
+      waves = w;
+    }
+  }
+  if (!int8_cache && hd == 128 && waves == 3) return 0;
+  return ct;
 }
 
 // Per range: 2 x num_q_heads partial records (head_dim + 2 floats each) and the 32-byte
@@ -475,38 +531,27 @@ int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_hea
                   ? 4
                   : 2;
   }
-  // Groups above 16 query heads: the wide kernel, one range per workgroup of four waves and one
-  // workgroup per CU, with as many column tiles per wave as its registers hold, spread evenly
-  // (5 tiles of 16: one wave at head_dim 64, 3 + 2 at 128), or fewer where the workgroups would
-  // otherwise hold under kWideMinUnits units of work each; under that even at two tiles per
-  // wave, and above head_dim 128 (one tile per wave), a wave per column tile as decode_kernel.
-  // 71 query heads on one kv head at 64, INT8, us before -> now (HIP-graph replays): B = 40 x 4096
-  // 41.2 -> 28.5, 40 x U[1, 8192] 43.2 -> 29.0, 8 x 4096 (3 + 2 tiles) 17.2 -> 16.7 (19.6 with 5);
-  // 16-bit cache 40 x 4096 30.0 -> 28.6; at 128: 64 heads on one, 16 x 8192 31.3 -> 27.7; 48 on
-  // two, 64 x U[1, 8192] 53.7 -> 47.9.
+  // Groups above 16 query heads: the wide kernel where it is the faster one (wide_column_tiles),
+  // one range per workgroup of four waves and one workgroup per CU.  INT8, us one wave per tile ->
+  // wide (HIP-graph replays): 71/1 heads at 64, 40 x 4096 35.1 -> 26.6, 8 x 32768 48.2 -> 32.7; 48/1
+  // at 128, 40 x 4096 37.2 -> 28.0.
   p.ct = 0;
   p.launch_ranges = num_ranges;
   p.launch_min_tiles = min_tiles;
-  const int32_t most = wide_most_tiles(hd);
-  if (p.col_tiles > 1 && !p.group_mode && most > 1) {
-    const int32_t tiles = p.col_tiles;
-    const double units = (double)batch * std::ceil((double)table_width * block_size / tile_tokens);
-    for (int32_t waves = (tiles + most - 1) / most; waves < tiles; ++waves) {
-      const int32_t heads = num_kv_heads * waves;  // workgroups per range
-      if (units * heads < (double)kWideMinUnits * cus) continue;
-      // ct tiles a wave may need fewer waves than were counted (5 tiles on 4 waves: 2 + 2 + 1):
-      // a workgroup without query heads would read the whole cache for nothing.
-      p.ct = (tiles + waves - 1) / waves;
-      p.col_tiles = (tiles + p.ct - 1) / p.ct;
-      p.grid_heads = num_kv_heads * p.col_tiles;
-      p.depth = 2;
-      p.halves = 1;
-      p.pair_min = 0x7fffffff;
-      if (auto_ranges_req)
-        p.launch_ranges = (int32_t)std::max<int64_t>(1, std::min<int64_t>(num_ranges, cus / p.grid_heads));
-      if (automatic) p.launch_min_tiles = std::max(min_tiles, kWideMinUnits);
-      break;
-    }
+  if (!p.group_mode) {
+    const double seq_tiles = std::ceil((double)table_width * block_size / tile_tokens);
+    p.ct = wide_column_tiles(i8, (flags & INT8KV_DECODE_QUANTIZE_Q) != 0, hd, p.col_tiles,
+                             num_kv_heads, seq_tiles, (double)batch * seq_tiles * num_kv_heads / cus);
+  }
+  if (p.ct > 0) {
+    p.col_tiles = (p.col_tiles + p.ct - 1) / p.ct;
+    p.grid_heads = num_kv_heads * p.col_tiles;
+    p.depth = 2;
+    p.halves = 1;
+    p.pair_min = 0x7fffffff;
+    if (auto_ranges_req)
+      p.launch_ranges = (int32_t)std::max<int64_t>(1, std::min<int64_t>(num_ranges, cus / p.grid_heads));
+    if (automatic) p.launch_min_tiles = std::max(min_tiles, kWideMinUnits);
   }
   // The layout above was chosen with the base charge; the plan itself charges what a sequence
   // start costs at the chosen depth (kSeqStartCost*).  decode_kernel and merge_kernel read the

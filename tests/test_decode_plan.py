@@ -379,6 +379,40 @@ def test_groups_above_16_leave_no_grid_head_empty():
     assert {(5, 2), (5, 3), (6, 2), (4, 2)} <= spread
 
 
+def test_column_tiles_per_wave():
+    """Groups above 16 at 256 CUs: column tiles per wave on both sides of each bound (units per CU,
+    longest sequence, shared workgroups, quantised queries, 16-bit caches)."""
+    def ct(units_per_cu, hq, hkv=1, d=64, tokens=8192, **kw):
+        """... with `units_per_cu` units of 32 tokens per compute unit and kv head set."""
+        batch = int(units_per_cu * 256 // (-(-tokens // 32) * hkv))
+        return _columns(batch=batch, hq=hq, hkv=hkv, d=d, width=tokens // 16, **kw)[0]
+
+    qq = dict(flags=_lib.DECODE_ALL | _lib.DECODE_QUANTIZE_Q)
+    # 5 tiles: 3 waves of 2 up to 8 units, 2 of 3 up to 18, then one of 5 (3 at head_dim 128).
+    assert [ct(u, 71) for u in (7, 8, 17, 18)] == [2, 3, 3, 5]
+    assert [ct(u, 71, tokens=2560) for u in (2.2, 1.6)] == [2, 0]  # 5 units a workgroup at least
+    assert [ct(u, 71, d=128) for u in (7, 8, 60)] == [2, 3, 3]
+    # 3 and 4 tiles move to a single workgroup at 12 and 30 units, 7 and 8 tiles to two at 12.
+    assert [ct(u, 48) for u in (11, 12)] == [2, 3] and [ct(u, 64) for u in (29, 30)] == [2, 4]
+    assert [ct(u, 112) for u in (11, 12)] == [2, 4] and [ct(u, 128) for u in (11, 12)] == [2, 4]
+    assert ct(60, 128, d=128) == 2  # (3 + 3 + 2 saves too little)
+    # Short sequences: 16 tiles, 32 where four waves of a workgroup share a kv head's lines.
+    assert [ct(20, 71, d=128, tokens=t) for t in (480, 512)] == [0, 3]
+    assert [ct(20, 64, d=128, tokens=t) for t in (992, 1024)] == [0, 2]
+    # Two tiles per kv head at 128, shared: 48 tiles and 40 units.
+    assert [ct(41, 40, 2, 128, t) for t in (1472, 1536)] == [0, 2]
+    assert [ct(u, 40, 2, 128) for u in (38, 40)] == [0, 2]
+    # Quantised queries at 128.
+    assert [ct(u, 64, d=128, **qq) for u in (31, 32)] == [0, 2]
+    assert [ct(u, 71, d=128, tokens=4096, **qq) for u in (5, 7)] == [0, 2]
+    assert ct(5, 71, **qq) == 2
+    # 16-bit caches: not three workgroups per range at 128, nor below 32 tiles there.
+    assert [ct(u, 71, d=128, cache=BF16) for u in (7, 8)] == [0, 3]
+    assert [ct(20, 71, d=128, tokens=t, cache=BF16) for t in (992, 1024)] == [0, 3]
+    # One tile per kv head, head_dim 256: never.
+    assert ct(40, 16) == 0 and ct(40, 64, d=256) == 0
+
+
 def test_plan_rejects_what_the_decode_rejects():
     for d in (8, 72, 100, 272, 512):  # head_dim: a multiple of 16 in [16, 256]
         with pytest.raises(_lib.Int8KVError, match="E_SHAPE"):

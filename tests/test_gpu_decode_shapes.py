@@ -23,6 +23,7 @@ import pytest
 import torch
 
 import int8kv
+from test_decode_plan import _columns as plan_columns
 from cases import bf16_caches, decode_case, oracle_int8, ranges_call, to_dev
 from conftest import MAX_ABS, MIN_COS, metrics
 from int8kv import _decode, _lib
@@ -246,13 +247,18 @@ def test_groups_above_16_several_tiles_per_wave(cuda, hq, hkv, d, cache):
     _check(out, ref, f"{hq}/{hkv} d={d} {cache}")
 
 
-# Calls of less work, whose column tiles are spread over more waves than registers would need: 5 as
-# 3 + 2 and 2 + 2 + 1, 6 as 2 + 2 + 2, 4 as 2 + 2 (query heads, kv heads, head_dim, batch, tokens).
+# Column tiles spread over the waves of one kv head: 2 + 2 + 1, 3 + 2 and 5; 2 + 2 + 2 and 3 + 3;
+# 2 + 2; 2 x 4 and 4 + 3; 2 + 1 and 3; a pair per kv head (query heads, kv heads, head_dim, batch, tokens,
+# tiles per wave on 256 compute units).
 @pytest.mark.parametrize("cache", ["int8", "bf16"])
-@pytest.mark.parametrize("hq,hkv,d,batch,tokens", [
-    (71, 1, 64, 2, 16384), (71, 1, 64, 5, 6144), (71, 1, 64, 7, 2560), (71, 1, 128, 7, 2560),
-    (96, 1, 64, 6, 2560), (64, 1, 64, 9, 2560), (34, 2, 128, 9, 2560)])
-def test_groups_above_16_spread_over_waves(cuda, hq, hkv, d, batch, tokens, cache):
+@pytest.mark.parametrize("hq,hkv,d,batch,tokens,per_wave", [
+    (71, 1, 64, 7, 2560, 2), (71, 1, 64, 9, 8192, 3), (71, 1, 64, 20, 8192, 5), (96, 1, 64, 6, 2560, 2),
+    (96, 1, 64, 9, 8192, 3), (64, 1, 64, 9, 2560, 2), (112, 1, 48, 9, 2560, 2), (112, 1, 48, 13, 8192, 4),
+    (48, 1, 128, 13, 4096, 2), (48, 1, 112, 13, 8192, 3), (50, 2, 64, 9, 2560, 2)])
+def test_groups_above_16_spread_over_waves(cuda, hq, hkv, d, batch, tokens, per_wave, cache):
+    columns = plan_columns(torch.int8 if cache == "int8" else torch.bfloat16, batch, hq, hkv, d,
+                           tokens // 16)
+    assert columns[0] == per_wave
     lens = [tokens] + [tokens - 37 * i for i in range(1, batch)]
     c = decode_case(lens, seed=hq + batch, hq=hq, hkv=hkv, head_dim=d, extra_blocks=5)
     q, kc, vc, bt, sl, ks, vs = to_dev(c, cuda)
