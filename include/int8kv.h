@@ -126,7 +126,10 @@ int int8kv_dynamic_cache_write(const void* key, const void* value, int src_dtype
  * takes kv heads in pairs (one wave per pair) and its automatic count is that of
  * num_kv_heads / 2; with more than 16 query heads per kv head each kv head takes
  * ceil(group / 16) waves (column tiles of 16 query heads) and the count is that of
- * num_kv_heads x ceil(group / 16).  int8kv_decode_workspace_bytes(..., 0) accounts for both.
+ * num_kv_heads x ceil(group / 16).  A workspace of that count is enough for num_ranges = 0.
+ * Where waves then hold several column tiles each, the token stream is cut into one range per
+ * workgroup and compute unit instead: mostly fewer, or, at head_dim up to 64, more if the workspace
+ * given holds them.  int8kv_decode_workspace_bytes(..., 0) accounts for all of this.
  */
 int32_t int8kv_decode_auto_ranges(int32_t num_kv_heads);
 
@@ -155,8 +158,9 @@ size_t int8kv_decode_workspace_bytes(int32_t num_q_heads, int32_t num_kv_heads, 
 typedef struct int8kv_decode_plan_t {
   int32_t layout;               /* INT8KV_LAYOUT_* */
   int32_t kernels;              /* kernel launches of a call with INT8KV_DECODE_ALL (0 for batch 0) */
-  int32_t num_ranges;           /* ranges layout: most ranges the token stream is cut into; every
-                                   layout: the range count the workspace is sized by */
+  int32_t num_ranges;           /* ranges layout: most ranges the token stream is cut into (groups
+                                   above 16 with num_ranges = 0: see int8kv_decode_auto_ranges);
+                                   every layout: the range count the call needs workspace for */
   int32_t min_tiles;            /* ranges layout: smallest range, in 32-token tiles */
   int32_t seq_cost;             /* ranges layout: stream units charged per sequence start */
   int32_t ranges_per_workgroup; /* ranges layout: 1, or 2 (paired ranges); 0 otherwise */
@@ -168,7 +172,8 @@ typedef struct int8kv_decode_plan_t {
   int32_t merge_waves;          /* waves per merge workgroup (0 without a merge) */
   int32_t merge_fold;           /* merge by sequence: records per lane slot and round */
   int32_t compute_units;        /* compute units the plan was made for */
-  uint64_t workspace_bytes;     /* workspace the call needs */
+  uint64_t workspace_bytes;     /* workspace of the call (num_ranges ranges, or the more it is cut
+                                   into: the call then accepts less, down to num_ranges) */
 } int8kv_decode_plan_t;
 
 /*

@@ -266,14 +266,18 @@ int32_t auto_ranges(int32_t num_kv_heads, int64_t cu) {
 }
 
 // Automatic range count of a shape: one wave per SIMD for the grid heads (a kv-head pair counts as
-// one); for the wide kernel (paged_decode_wide.h) at least one workgroup per CU.
-int32_t auto_ranges_for(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, bool pair,
-                        int64_t cu) {
+// one).
+int32_t auto_ranges_for(int32_t num_q_heads, int32_t num_kv_heads, bool pair, int64_t cu) {
+  return auto_ranges(pair ? num_kv_heads / 2 : grid_heads(num_q_heads, num_kv_heads), cu);
+}
+
+// Most ranges the wide kernel (paged_decode_wide.h) launches with automatically: one workgroup per
+// CU with as few waves per kv head as it takes.  More than the count above for 5 column tiles at
+// head_dim 64 (71 heads on one: 256 against 204); 0 for shapes without that kernel.
+int32_t wide_auto_ranges(int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, int64_t cu) {
   const int32_t tiles = col_tiles(num_q_heads, num_kv_heads);
-  const int32_t r = auto_ranges(pair ? num_kv_heads / 2 : num_kv_heads * tiles, cu);
   const int32_t most = wide_most_tiles(padded_head_dim(head_dim));
-  if (tiles == 1 || most == 1) return r;
-  return std::max(r, (int32_t)(cu / (num_kv_heads * ((tiles + most - 1) / most))));
+  return tiles == 1 || most == 1 ? 0 : (int32_t)(cu / (num_kv_heads * ((tiles + most - 1) / most)));
 }
 
 // Column tiles per wave of the wide kernel (paged_decode_wide.h) for a range-layout call with
@@ -373,9 +377,12 @@ extern "C" size_t int8kv_decode_workspace_bytes(int32_t num_q_heads, int32_t num
   if (!shape_ok(num_q_heads, num_kv_heads, head_dim, block_size) || num_ranges < 0 ||
       num_ranges > kMaxRangesLimit)
     return 0;
-  if (num_ranges == 0)
-    num_ranges = auto_ranges_for(num_q_heads, num_kv_heads, head_dim,
-                                 kv_pair_shape(num_q_heads, num_kv_heads, head_dim), cu_count());
+  if (num_ranges == 0) {
+    const int64_t cu = cu_count();
+    num_ranges = std::max(auto_ranges_for(num_q_heads, num_kv_heads,
+                                          kv_pair_shape(num_q_heads, num_kv_heads, head_dim), cu),
+                          wide_auto_ranges(num_q_heads, num_kv_heads, head_dim, cu));
+  }
   return workspace_bytes(num_q_heads, num_ranges, padded_head_dim(head_dim));
 }
 
@@ -441,12 +448,13 @@ void merge_shape(int64_t batch, int64_t table_width, int32_t block_size, int32_t
 // The host's whole decision for one call (argument checks on sizes and dtypes included; no
 // pointer is looked at).  cus: compute units of the device the call runs on.  scratch_cap: the
 // no-allocation entry point's workspace limit (0 = none); an automatic range count is lowered
-// to fit it.
+// to fit it.  workspace_cap: the workspace there is; the wide kernel's automatic ranges may exceed the
+// automatic count (which is what a call needs at least) where it holds them.
 int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_heads,
               int32_t num_kv_heads, int32_t head_dim, int64_t num_blocks, int32_t block_size,
               int64_t table_width, int64_t key_head_stride, int64_t value_head_stride,
               int32_t num_ranges, int32_t min_tiles, uint32_t flags, int64_t cus,
-              size_t scratch_cap, HostPlan* hp) {
+              size_t scratch_cap, size_t workspace_cap, HostPlan* hp) {
   if (query_dtype != INT8KV_F32 && query_dtype != INT8KV_F16 && query_dtype != INT8KV_BF16)
     return INT8KV_E_DTYPE;
   if (cache_dtype != INT8KV_I8 && cache_dtype != INT8KV_BF16 && cache_dtype != INT8KV_F16)
@@ -470,7 +478,7 @@ int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_hea
                           key_head_stride == head_dim && value_head_stride == head_dim;
   const int32_t wave_heads = kv_pair_ok ? num_kv_heads / 2 : hv;  // per range
   if (num_ranges == 0)
-    num_ranges = auto_ranges_for(num_q_heads, num_kv_heads, head_dim, kv_pair_ok, cus);
+    num_ranges = auto_ranges_for(num_q_heads, num_kv_heads, kv_pair_ok, cus);
   if (scratch_cap > 0 && auto_ranges_req) {
     // The partials of the automatic count may exceed the fixed scratch array (large GQA groups
     // or head_dim 256): take the most ranges it holds instead.
@@ -549,10 +557,15 @@ int plan_call(int query_dtype, int cache_dtype, int64_t batch, int32_t num_q_hea
     p.depth = 2;
     p.halves = 1;
     p.pair_min = 0x7fffffff;
-    if (auto_ranges_req)
-      p.launch_ranges = (int32_t)std::max<int64_t>(1, std::min<int64_t>(num_ranges, cus / p.grid_heads));
+    if (auto_ranges_req) {
+      const size_t fit = std::min<size_t>(workspace_cap / workspace_bytes(num_q_heads, 1, hd),
+                                          kMaxRangesLimit);
+      p.launch_ranges = (int32_t)std::max<int64_t>(
+          1, std::min<int64_t>(std::max<int64_t>(num_ranges, (int64_t)fit), cus / p.grid_heads));
+    }
     if (automatic) p.launch_min_tiles = std::max(min_tiles, kWideMinUnits);
   }
+  p.record_ranges = std::max(num_ranges, p.launch_ranges);
   // The layout above was chosen with the base charge; the plan itself charges what a sequence
   // start costs at the chosen depth (kSeqStartCost*).  decode_kernel and merge_kernel read the
   // same value, so their range bounds agree.
@@ -628,13 +641,14 @@ int decode_entry(
     return INT8KV_E_NULL;
   if (table_dtype != INT8KV_I32 && table_dtype != INT8KV_I64) return INT8KV_E_DTYPE;
   if (seq_lens_dtype != INT8KV_I32 && seq_lens_dtype != INT8KV_I64) return INT8KV_E_DTYPE;
+  if (from_scratch) workspace_bytes_given = kScratchBytes;
   HostPlan hp;
   {
     // Sizes and dtypes first (the plan checks them); the CU count only once they pass.
     const int st = plan_call(query_dtype, cache_dtype, batch, num_q_heads, num_kv_heads, head_dim,
                              num_blocks, block_size, table_width, key_cache_strides[2],
                              value_cache_strides[2], num_ranges, min_tiles, flags, 256,
-                             from_scratch ? kScratchBytes : 0, &hp);
+                             from_scratch ? kScratchBytes : 0, workspace_bytes_given, &hp);
     if (st != INT8KV_OK) return st;
   }
   if (batch == 0) return INT8KV_OK;
@@ -659,13 +673,12 @@ int decode_entry(
     const int st = plan_call(query_dtype, cache_dtype, batch, num_q_heads, num_kv_heads, head_dim,
                              num_blocks, block_size, table_width, key_cache_strides[2],
                              value_cache_strides[2], num_ranges, min_tiles, flags, cu_count(),
-                             from_scratch ? kScratchBytes : 0, &hp);
+                             from_scratch ? kScratchBytes : 0, workspace_bytes_given, &hp);
     if (st != INT8KV_OK) return st;
   }
   if (from_scratch) {
     const int st = current_scratch(&workspace);
     if (st != INT8KV_OK) return st;
-    workspace_bytes_given = kScratchBytes;
   }
   if (workspace == nullptr || workspace_bytes_given < hp.need || ((uintptr_t)workspace % 16) != 0)
     return INT8KV_E_WORKSPACE;
@@ -691,7 +704,7 @@ int decode_entry(
   a.out = static_cast<char*>(out);
   a.o_sb = out_strides[0];
   a.o_sh = out_strides[1];
-  const int64_t recs = (int64_t)hp.num_ranges * 2 * num_q_heads;
+  const int64_t recs = (int64_t)hp.record_ranges * 2 * num_q_heads;
   float* ws = static_cast<float*>(workspace);
   a.ws_acc = ws;
   a.ws_m = ws + recs * hp.hd;
@@ -753,7 +766,7 @@ extern "C" int int8kv_decode_plan(int query_dtype, int cache_dtype, int64_t batc
   const int st = plan_call(query_dtype, cache_dtype, batch, num_q_heads, num_kv_heads, head_dim,
                            num_blocks, block_size, table_width, key_head_stride,
                            value_head_stride, num_ranges, min_tiles, flags, cus,
-                           no_alloc ? kScratchBytes : 0, &hp);
+                           no_alloc ? kScratchBytes : 0, no_alloc ? kScratchBytes : SIZE_MAX, &hp);
   if (st != INT8KV_OK) return st;
   int8kv_decode_plan_t p{};
   p.layout = !hp.group_mode ? INT8KV_LAYOUT_RANGES
@@ -761,7 +774,7 @@ extern "C" int int8kv_decode_plan(int query_dtype, int cache_dtype, int64_t batc
                             : INT8KV_LAYOUT_PER_SEQUENCE;
   p.kernels = batch == 0 ? 0 : (hp.merge == kMergeNone ? 1 : 2);
   p.num_ranges = hp.num_ranges;
-  p.min_tiles = hp.min_tiles;
+  p.min_tiles = hp.launch_min_tiles;
   p.seq_cost = hp.seq_cost;
   p.ranges_per_workgroup = hp.group_mode ? 0 : hp.halves;
   p.depth = hp.launch_depth;
@@ -772,24 +785,24 @@ extern "C" int int8kv_decode_plan(int query_dtype, int cache_dtype, int64_t batc
   p.merge_waves = hp.merge_waves;
   p.merge_fold = hp.merge_fold;
   p.compute_units = (int32_t)cus;
-  p.workspace_bytes = hp.need;
+  p.workspace_bytes = workspace_bytes(num_q_heads, hp.record_ranges, hp.hd);
   *plan = p;
   return INT8KV_OK;
 }
 
 // How the range layout's launch spreads groups above 16 query heads, for the planner's tests (not
-// part of the public C ABI).  columns: column tiles of 16 query heads per wave (0: one wave per
+// part of the public C ABI) and with `workspace` bytes given.  columns: column tiles of 16 query heads per wave (0: one wave per
 // tile), grid heads, ranges and smallest range launched.
 extern "C" int int8kv_decode_plan_columns(int query_dtype, int cache_dtype, int64_t batch,
                                           int32_t num_q_heads, int32_t num_kv_heads,
                                           int32_t head_dim, int64_t num_blocks, int32_t block_size,
                                           int64_t table_width, int32_t num_ranges,
                                           int32_t min_tiles, uint32_t flags, int32_t compute_units,
-                                          int32_t columns[4]) {
+                                          size_t workspace, int32_t columns[4]) {
   HostPlan hp;
   const int st = plan_call(query_dtype, cache_dtype, batch, num_q_heads, num_kv_heads, head_dim,
                            num_blocks, block_size, table_width, head_dim, head_dim, num_ranges,
-                           min_tiles, flags, compute_units, 0, &hp);
+                           min_tiles, flags, compute_units, 0, workspace, &hp);
   if (st != INT8KV_OK) return st;
   columns[0] = hp.ct;
   columns[1] = hp.grid_heads;

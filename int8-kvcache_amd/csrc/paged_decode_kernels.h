@@ -1914,7 +1914,7 @@ enum MergeKind { kMergeNone = 0, kMergeBySequence = 1, kMergeByRange = 2, kMerge
 // (no device memory is read): int8kv_paged_decode launches from it and int8kv_decode_plan
 // reports it.
 struct HostPlan {
-  int32_t num_ranges;   // range count upper bound (the workspace's records are sized by it)
+  int32_t num_ranges;   // range count upper bound (the least workspace is sized by it)
   int32_t min_tiles;
   bool group_mode;      // per-sequence workgroups (split or not)
   int32_t split;        // split layout: workgroups per (sequence, kv head); 0 = not split
@@ -1935,10 +1935,11 @@ struct HostPlan {
   int32_t grid_heads;   // kv heads x col_tiles
   int32_t col_tiles;    // MFMA column tiles of 16 query heads per kv head
   int32_t ct;           // column tiles per wave (paged_decode_wide.h); 0: one grid head per wave
-  int32_t launch_ranges;  // ranges the kernels run with (num_ranges, or fewer with ct)
+  int32_t launch_ranges;  // ranges the kernels run with (num_ranges; with ct one workgroup per CU)
   int32_t launch_min_tiles;
+  int32_t record_ranges;  // ranges the workspace's records are laid out for
   int64_t cus;
-  size_t need;          // workspace bytes
+  size_t need;          // least workspace bytes
 };
 
 // Most column tiles of 16 query heads that one wave of the wide range kernel holds

@@ -108,7 +108,7 @@ def bind(path: Path) -> ctypes.CDLL:
     lib.int8kv_decode_plan_columns.restype = ctypes.c_int
     lib.int8kv_decode_plan_columns.argtypes = [
         ctypes.c_int, ctypes.c_int, i64, i32, i32, i32, i64, i32, i64, i32, i32, u32, i32,
-        ctypes.POINTER(i32),
+        sz, ctypes.POINTER(i32),
     ]
     lib.int8kv_paged_decode.restype = ctypes.c_int
     lib.int8kv_paged_decode.argtypes = [

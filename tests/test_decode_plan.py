@@ -352,12 +352,12 @@ def test_groups_above_16_take_column_tiles():
 
 
 def _columns(cache=I8, batch=1, hq=64, hkv=1, d=64, width=32, cus=256, bs=16, query=Q, ranges=0,
-             min_tiles=0, flags=_lib.DECODE_ALL):
+             min_tiles=0, flags=_lib.DECODE_ALL, workspace=1 << 40):
     """(column tiles per wave, grid heads, ranges, smallest range) of the range layout's launch."""
     out = (ctypes.c_int32 * 4)()
     _lib.check(_lib.load().int8kv_decode_plan_columns(
         _lib.DTYPE_CODE[query], _lib.DTYPE_CODE[cache], batch, hq, hkv, d, batch * width + 16, bs,
-        width, ranges, min_tiles, flags, cus, out), "int8kv_decode_plan_columns")
+        width, ranges, min_tiles, flags, cus, workspace, out), "int8kv_decode_plan_columns")
     return tuple(out)
 
 
@@ -377,6 +377,26 @@ def test_groups_above_16_leave_no_grid_head_empty():
                         assert waves == -(-tiles // max(ct, 1)), (group, hkv, d, batch, width, ct, heads)
                         spread.add((tiles, ct))
     assert {(5, 2), (5, 3), (6, 2), (4, 2)} <= spread
+
+
+def test_groups_above_16_ranges_follow_the_workspace():
+    """71 query heads on one kv head at head_dim 64: the automatic count is that of 5 kv heads, and
+    a workspace of it is enough; the kernel that takes all five tiles per wave launches a range
+    per compute unit where the workspace holds as many.  The plan's smallest range is the launch's."""
+    per = _per_range(71, 64)
+    kw = dict(batch=40, hq=71, d=64, width=256)
+    p = plan(hkv=1, **kw)
+    assert p["num_ranges"] == 4 * 256 // 5 == 204
+    assert p["workspace_bytes"] == 256 * per
+    assert p["min_tiles"] == 8
+    assert _columns(**kw) == (5, 1, 256, 8)
+    assert _columns(workspace=256 * per, **kw)[2] == 256
+    assert _columns(workspace=250 * per + 1, **kw)[2] == 250
+    assert _columns(workspace=204 * per, **kw)[2] == 204
+    assert _columns(ranges=300, **kw)[2] == 300 and _columns(ranges=100, **kw)[2] == 100
+    # Not that kernel (sequences under 16 tiles): the automatic count alone.
+    p = plan(hkv=1, batch=400, hq=71, d=64, width=20)
+    assert (p["num_ranges"], p["workspace_bytes"]) == (204, 204 * per)
 
 
 def test_column_tiles_per_wave():

@@ -275,6 +275,35 @@ def test_groups_above_16_spread_over_waves(cuda, hq, hkv, d, batch, tokens, per_
     _check(out, ref, f"{cache} {hq}/{hkv} d={d} {batch}x{tokens}")
 
 
+def test_groups_above_16_with_the_automatic_counts_workspace(cuda):
+    """71 heads on one kv head at 64: a workspace of the automatic count's ranges (those of 5 kv
+    heads), of any more, and one byte too few."""
+    c = decode_case([4000 - 7 * i for i in range(40)], seed=5, hq=71, hkv=1, head_dim=64)
+    q, kc, vc, bt, sl, ks, vs = to_dev(c, cuda)
+    lib, ref = _lib.load(), oracle_int8(c)
+    least = lib.int8kv_decode_workspace_bytes(71, 1, 64, 16, lib.int8kv_decode_auto_ranges(5))
+    full = lib.int8kv_decode_workspace_bytes(71, 1, 64, 16, 0)
+    assert full > least
+    for given in (full, (full + least) // 2, least, least - 1):
+        work = torch.full((full + 4096,), 0x5A, dtype=torch.uint8, device=cuda)
+        out = torch.full_like(q, float("nan"))
+        status = lib.int8kv_paged_decode(
+            q.data_ptr(), _lib.DTYPE_CODE[q.dtype], 40, 71, 64, _lib.strides(q), kc.data_ptr(),
+            vc.data_ptr(), _lib.I8, kc.shape[0], 16, 1, _lib.strides(kc), _lib.strides(vc), bt.data_ptr(),
+            _lib.DTYPE_CODE[bt.dtype], bt.shape[1], _lib.strides(bt), sl.data_ptr(),
+            _lib.DTYPE_CODE[sl.dtype], ks.data_ptr(), vs.data_ptr(), 64**-0.5, out.data_ptr(),
+            _lib.strides(out), work.data_ptr(), given, 0, 0, _lib.DECODE_ALL, _lib.stream_handle(cuda))
+        torch.cuda.synchronize()
+        if given < least:
+            with pytest.raises(_lib.Int8KVError, match="E_WORKSPACE"):
+                _lib.check(status, "int8kv_paged_decode")
+            assert torch.isnan(out).all()
+            continue
+        assert status == 0
+        _check(out, ref, f"workspace {given}")
+        assert (work[given:] == 0x5A).all(), "written past the workspace"
+
+
 @pytest.mark.parametrize("cache", ["int8", "bf16"])
 @pytest.mark.parametrize("hq,hkv,d", [(14, 2, 64), (28, 4, 128), (16, 8, 256)])
 def test_one_tile_per_wave_bound(cuda, hq, hkv, d, cache):
