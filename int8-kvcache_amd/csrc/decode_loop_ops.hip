@@ -153,51 +153,73 @@ __global__ __launch_bounds__(kRopeThreads) void rotary_kernel(
 }
 
 constexpr int kActThreads = 256;
-constexpr int kActUnroll = 2;  // 16-byte pieces of a row per thread (4: the same; 1: 130 us below)
 constexpr double kInfinityCacheBytes = 256.0 * 1024 * 1024;
 
-// 2^shift threads per row (256 from 2048 columns on), kActUnroll pieces of 8 columns each; a row
-// of more pieces takes wgs_per_row workgroups.  The gate and up values are streamed once: read
-// with the non-temporal hint; the result is stored with it (NT_OUT) when the call's bytes exceed
-// the 256 MB Infinity Cache, so that what the next product could find there is not pushed out by
-// what it could not.  6007 x 18944 (683 MB): 150 us, 4.6 TB/s, with a 64-bit division per lane,
-// expf, the IEEE divide and plain accesses (VALU-bound); 134.7 us without those; 115.4 us, 5.9
-// TB/s, with the hint on the stores too.
-template <bool NT_OUT>
+// Division of n < 2^31 by a value known to the host: n / d = n mul >> (31 + shift), exact since
+// mul d - 2^(31 + shift) < d <= 2^shift.
+struct Divisor {
+  uint32_t mul;
+  int shift;
+  __device__ __forceinline__ uint32_t operator()(uint32_t n) const {
+    return (uint32_t)(((uint64_t)n * mul) >> (31 + shift));
+  }
+};
+
+Divisor divisor(uint32_t d) {
+  int shift = 0;
+  while (((uint64_t)1 << shift) < d) ++shift;
+  return {(uint32_t)((((uint64_t)1 << (31 + shift)) + d - 1) / d), shift};
+}
+
+// 16-byte pieces (8 columns) of the call's `total` (fewer than 2^31) per thread, whatever the width:
+// with whole workgroups per row the 608 pieces of ffn 4864 took two of 512.  Bound by HBM, or by
+// the caches that the product before has left gate and up in.
+// NT: the call's bytes exceed the 256 MB Infinity Cache.  Gate and up are then read and the result is
+// stored with the non-temporal hint, so that what the next product could find in the cache is not pushed
+// out by what it could not, two pieces per thread.  Smaller calls take plain accesses, since reading
+// past the caches costs (2048 x 4864, 60 MB: 10.8 us, with the hint on the loads 17.9), and one
+// piece per thread (32 x 18944: 2.38 us against 2.66 with two).
+// 6007 x 18944 (683 MB): 150 us, 4.6 TB/s, with a 64-bit division per lane, expf, the IEEE divide
+// and plain accesses (VALU-bound); 134.7 us without those; 115.4 us, 5.9 TB/s, with the hint.
+template <bool NT>
 __global__ __launch_bounds__(kActThreads) void silu_mul_kernel(
-    const uint16_t* __restrict__ gu, uint16_t* __restrict__ out, int64_t rows, int ffn, int64_t is,
-    int64_t os, uint32_t wgs_per_row, int shift) {
-  const uint32_t group = blockIdx.x / wgs_per_row;
-  const int64_t row = ((int64_t)group << (8 - shift)) + (threadIdx.x >> shift);
-  if (row >= rows) return;
-  const int lanes = 1 << shift;
-  const int c0 = (int)(blockIdx.x - group * wgs_per_row) * kActThreads * kActUnroll +
-                 (int)(threadIdx.x & (lanes - 1));
-  const uint16_t* src = gu + row * is;
-  u32x4 gw[kActUnroll], uw[kActUnroll];
+    const uint16_t* __restrict__ gu, uint16_t* __restrict__ out, uint32_t total, int ffn, int64_t is,
+    int64_t os, Divisor per_row) {
+  constexpr int kPieces = NT ? 2 : 1;
+  const uint32_t t0 = blockIdx.x * (uint32_t)(kActThreads * kPieces) + threadIdx.x;
+  u32x4 gw[kPieces], uw[kPieces];
+  u32x4* dst[kPieces];
 #pragma unroll
-  for (int j = 0; j < kActUnroll; ++j) {
-    const int c = 8 * (c0 + j * lanes);
-    if (c < ffn) {
-      gw[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + c));
-      uw[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src + ffn + c));
+  for (int j = 0; j < kPieces; ++j) {
+    const uint32_t t = t0 + j * kActThreads;
+    if (t < total) {
+      const uint32_t row = per_row(t);
+      const int64_t c = 8 * (int64_t)(t - row * (uint32_t)(ffn / 8));
+      const u32x4* g = reinterpret_cast<const u32x4*>(gu + row * is + c);
+      const u32x4* u = reinterpret_cast<const u32x4*>(gu + row * is + ffn + c);
+      if constexpr (NT) {
+        gw[j] = __builtin_nontemporal_load(g);
+        uw[j] = __builtin_nontemporal_load(u);
+      } else {
+        gw[j] = *g;
+        uw[j] = *u;
+      }
+      dst[j] = reinterpret_cast<u32x4*>(out + row * os + c);
     }
   }
 #pragma unroll
-  for (int j = 0; j < kActUnroll; ++j) {
-    const int c = 8 * (c0 + j * lanes);
-    if (c >= ffn) break;
+  for (int j = 0; j < kPieces; ++j) {
+    if (t0 + j * kActThreads >= total) break;
     float g[8], u[8], y[8];
     unpack(gw[j], g);
     unpack(uw[j], u);
     silu(g, y);
 #pragma unroll
     for (int i = 0; i < 8; ++i) y[i] = round_bf16(y[i]) * u[i];
-    u32x4* dst = reinterpret_cast<u32x4*>(out + row * os + c);
-    if constexpr (NT_OUT)
-      __builtin_nontemporal_store(pack8(y), dst);
+    if constexpr (NT)
+      __builtin_nontemporal_store(pack8(y), dst[j]);
     else
-      *dst = pack8(y);
+      *dst[j] = pack8(y);
   }
 }
 
@@ -518,22 +540,20 @@ extern "C" int int8kv_silu_mul(const void* gate_up, void* out, int64_t rows, int
       gate_up_row_stride < 2 * static_cast<int64_t>(ffn) || out_row_stride < ffn)
     return INT8KV_E_STRIDE;
   if (rows == 0) return INT8KV_OK;
-  const int pieces = ffn / 8;
-  int shift = 0;
-  while (shift < 8 && (kActUnroll << shift) < pieces) ++shift;
-  const int64_t per_row = shift < 8 ? 1 : (pieces + kActThreads * kActUnroll - 1) / (kActThreads * kActUnroll);
-  const int64_t rows_per_wg = kActThreads >> shift;
-  // (A grid holds 2^31 - 1 workgroups; more rows than that take several launches.)
-  const int64_t most_rows = 0x7fffffff / per_row * rows_per_wg;
+  const int64_t pieces = ffn / 8;
+  const bool streams = 6.0 * rows * ffn > kInfinityCacheBytes;
+  const int64_t per_wg = kActThreads * (streams ? 2 : 1);
+  // (The kernel counts pieces in 31 bits; more than that take several launches.)
+  const int64_t most_rows = (0x7fffffff - per_wg) / pieces;
+  auto kernel = streams ? silu_mul_kernel<true> : silu_mul_kernel<false>;
   for (int64_t r0 = 0; r0 < rows; r0 += most_rows) {
-    const int64_t n = rows - r0 < most_rows ? rows - r0 : most_rows;
-    const int64_t wgs = (n + rows_per_wg - 1) / rows_per_wg * per_row;
-    auto kernel = 6.0 * rows * ffn > kInfinityCacheBytes ? silu_mul_kernel<true> : silu_mul_kernel<false>;
-    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>(wgs)), dim3(kActThreads), 0,
-                       static_cast<hipStream_t>(stream),
+    const int64_t total = (rows - r0 < most_rows ? rows - r0 : most_rows) * pieces;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<uint32_t>((total + per_wg - 1) / per_wg)),
+                       dim3(kActThreads), 0, static_cast<hipStream_t>(stream),
                        static_cast<const uint16_t*>(gate_up) + r0 * gate_up_row_stride,
-                       static_cast<uint16_t*>(out) + r0 * out_row_stride, n, static_cast<int>(ffn),
-                       gate_up_row_stride, out_row_stride, static_cast<uint32_t>(per_row), shift);
+                       static_cast<uint16_t*>(out) + r0 * out_row_stride,
+                       static_cast<uint32_t>(total), static_cast<int>(ffn), gate_up_row_stride,
+                       out_row_stride, divisor(static_cast<uint32_t>(pieces)));
   }
   return status(hipGetLastError());
 }

@@ -114,6 +114,45 @@ def test_silu_mul(cuda, rows, ffn):
     assert (out.float() - unfused.float()).abs().max().item() <= float(tol.max())
 
 
+@pytest.mark.parametrize("rows,ffn", [(1, 4096), (2, 4104), (37, 4864), (300, 8), (700, 2056), (6, 40)])
+def test_silu_mul_pieces_across_rows(cuda, rows, ffn):
+    """Widths below, at and above a workgroup's pieces, rows that start inside one, strided
+    rows: each row as by itself, and nothing past the width."""
+    g = torch.Generator(device=cuda).manual_seed(ffn)
+    wide = (torch.randn(rows, 2 * ffn + 24, generator=g, device=cuda) * 4).to(torch.bfloat16)
+    out = torch.full((rows + 1, ffn + 16), float("nan"), dtype=torch.bfloat16, device=cuda)
+    DL.hip_silu_mul(wide[:, : 2 * ffn], out[:rows, :ffn])
+    assert torch.isnan(out[rows]).all() and torch.isnan(out[:, ffn:]).all()
+    one = torch.empty(1, ffn, dtype=torch.bfloat16, device=cuda)
+    for r in {0, 1, rows // 2, rows - 1} & set(range(rows)):
+        assert torch.equal(DL.hip_silu_mul(wide[r : r + 1, : 2 * ffn].clone(), one)[0], out[r, :ffn])
+
+
+def test_silu_mul_streamed(cuda):
+    """Calls past the Infinity Cache's size (non-temporal accesses) equal smaller ones bit for bit."""
+    g = torch.Generator(device=cuda).manual_seed(4)
+    gu = (torch.randn(9001, 2 * 5000, generator=g, device=cuda) * 4).to(torch.bfloat16)
+    out = DL.hip_silu_mul(gu, torch.empty(9001, 5000, dtype=torch.bfloat16, device=cuda))
+    part = torch.empty(1500, 5000, dtype=torch.bfloat16, device=cuda)
+    for r in (0, 3333, 7501):
+        assert torch.equal(DL.hip_silu_mul(gu[r : r + 1500], part), out[r : r + 1500])
+
+
+def test_silu_mul_of_the_widest_row(cuda):
+    """ffn = 2^31 - 8, whose byte offsets and piece counts leave 32 bits: both ends of the row."""
+    ffn = 2**31 - 8
+    gu = torch.zeros(1, 2 * ffn, dtype=torch.bfloat16, device=cuda)
+    out = torch.full((1, ffn + 4096), 7.0, dtype=torch.bfloat16, device=cuda)
+    g = torch.Generator(device=cuda).manual_seed(8)
+    ends = (torch.randn(4, 4096, generator=g, device=cuda) * 4).to(torch.bfloat16)
+    gu[0, :4096], gu[0, ffn - 4096 : ffn] = ends[0], ends[1]
+    gu[0, ffn : ffn + 4096], gu[0, 2 * ffn - 4096 :] = ends[2], ends[3]
+    DL.hip_silu_mul(gu, out[:, :ffn])
+    ref = DL.hip_silu_mul(torch.cat([ends[:2], ends[2:]], dim=1), torch.empty_like(ends[:2]))
+    assert torch.equal(out[0, :4096], ref[0]) and torch.equal(out[0, ffn - 4096 : ffn], ref[1])
+    assert (out[0, ffn:] == 7).all() and not out[0, 4096 : ffn - 4096].any()
+
+
 def test_strided_rows(cuda):
     """Row strides larger than the row (views into wider buffers) are honoured."""
     g = torch.Generator().manual_seed(9)
