@@ -101,35 +101,42 @@ __global__ __launch_bounds__(kNormThreads) void add_rms_norm_kernel(
   }
 }
 
+// Division of n < 2^31 by a value known to the host: n / d = n mul >> (31 + shift), exact since
+// mul d - 2^(31 + shift) < d <= 2^shift.
+struct Divisor {
+  uint32_t mul;
+  int shift;
+  __device__ __forceinline__ uint32_t operator()(uint32_t n) const {
+    return (uint32_t)(((uint64_t)n * mul) >> (31 + shift));
+  }
+};
+
+Divisor divisor(uint32_t d) {
+  int shift = 0;
+  while (((uint64_t)1 << shift) < d) ++shift;
+  return {(uint32_t)((((uint64_t)1 << (31 + shift)) + d - 1) / d), shift};
+}
+
 constexpr int kRopeThreads = 256;
 
-// One thread per (row, head, 8-pair chunk).  A workgroup takes 256 of a row's chunks, or, where a
-// row has fewer, 256 / per_row whole rows: the row then costs a scalar or a 32-bit division
-// instead of a 64-bit one per lane (~100 instructions).  6007 rows x 32 heads x 128: 23.4 ->
-// 17.9 us (5.8 TB/s).
+// One thread per (row, head, 8-pair chunk), counted over the call's `total` chunks (fewer than
+// 2^31): whatever the head count, workgroups are full (40 heads x 128 have 320 chunks a row; with whole
+// workgroups per row 2048 rows took 10.8 us, 7.7 before that).  `step` chunks per workgroup: 256, or
+// whole rows where those leave under a sixteenth of it idle (a row's lines then belong to one
+// XCD: 6007 rows x 3 x 48 2.85 -> 2.56 us).  Bound by HBM: a multiplication
+// for the row instead of a 64-bit division per lane (~100 instructions): 6007 rows x 32 heads x 128
+// 23.4 -> 17.9 us (5.8 TB/s).
 __global__ __launch_bounds__(kRopeThreads) void rotary_kernel(
-    uint16_t* __restrict__ qkv, int64_t rows, int64_t row_stride, int num_heads, int head_dim,
+    uint16_t* __restrict__ qkv, uint32_t total, int64_t row_stride, int head_dim,
     const int64_t* __restrict__ positions, const float* __restrict__ cos_t,
-    const float* __restrict__ sin_t, int64_t max_pos, uint32_t wgs_per_row) {
-  const int chunks = head_dim / 16;  // 8 rotation pairs per thread
-  const uint32_t per_row = (uint32_t)(num_heads * chunks);
-  int64_t row;
-  uint32_t rem;
-  if (per_row >= kRopeThreads) {
-    const uint32_t r = blockIdx.x / wgs_per_row;
-    row = r;
-    rem = (blockIdx.x - r * wgs_per_row) * kRopeThreads + threadIdx.x;
-    if (rem >= per_row) return;
-  } else {
-    const uint32_t rows_per_wg = kRopeThreads / per_row;
-    const uint32_t r = threadIdx.x / per_row;
-    if (r >= rows_per_wg) return;
-    row = (int64_t)blockIdx.x * rows_per_wg + r;
-    rem = threadIdx.x - r * per_row;
-  }
-  if (row >= rows) return;
-  const int head = (int)rem / chunks;
-  const int c = (int)rem - head * chunks;
+    const float* __restrict__ sin_t, int64_t max_pos, uint32_t step, uint32_t per_row,
+    Divisor by_row, Divisor by_chunk) {
+  const uint32_t t = blockIdx.x * step + threadIdx.x;
+  if (threadIdx.x >= step || t >= total) return;
+  const int64_t row = by_row(t);
+  const uint32_t rem = t - (uint32_t)row * per_row;
+  const int head = (int)by_chunk(rem);
+  const int c = (int)(rem - (uint32_t)head * (uint32_t)(head_dim / 16));  // 8 rotation pairs per thread
   const int64_t p = positions[row];
   if (p < 0 || p >= max_pos) return;
   const int half = head_dim / 2;
@@ -154,22 +161,6 @@ __global__ __launch_bounds__(kRopeThreads) void rotary_kernel(
 
 constexpr int kActThreads = 256;
 constexpr double kInfinityCacheBytes = 256.0 * 1024 * 1024;
-
-// Division of n < 2^31 by a value known to the host: n / d = n mul >> (31 + shift), exact since
-// mul d - 2^(31 + shift) < d <= 2^shift.
-struct Divisor {
-  uint32_t mul;
-  int shift;
-  __device__ __forceinline__ uint32_t operator()(uint32_t n) const {
-    return (uint32_t)(((uint64_t)n * mul) >> (31 + shift));
-  }
-};
-
-Divisor divisor(uint32_t d) {
-  int shift = 0;
-  while (((uint64_t)1 << shift) < d) ++shift;
-  return {(uint32_t)((((uint64_t)1 << (31 + shift)) + d - 1) / d), shift};
-}
 
 // 16-byte pieces (8 columns) of the call's `total` (fewer than 2^31) per thread, whatever the width:
 // with whole workgroups per row the 608 pieces of ffn 4864 took two of 512.  Bound by HBM, or by
@@ -518,16 +509,21 @@ extern "C" int int8kv_rotary_inplace(void* qkv, int64_t rows, int64_t row_stride
     return INT8KV_E_STRIDE;
   if (rows == 0) return INT8KV_OK;
   const int64_t per_row = static_cast<int64_t>(num_heads) * (head_dim / 16);
-  if (per_row > 0x3fffffff) return INT8KV_E_SHAPE;
-  const int64_t wgs_per_row = (per_row + kRopeThreads - 1) / kRopeThreads;
-  const int64_t rows_per_wg = per_row >= kRopeThreads ? 1 : kRopeThreads / per_row;
-  const int64_t blocks = (rows + rows_per_wg - 1) / rows_per_wg * wgs_per_row;
-  if (blocks > 0x7fffffff) return INT8KV_E_SHAPE;
-  hipLaunchKernelGGL(rotary_kernel, dim3(static_cast<uint32_t>(blocks)), dim3(kRopeThreads), 0,
-                     static_cast<hipStream_t>(stream), static_cast<uint16_t*>(qkv), rows,
-                     row_stride, static_cast<int>(num_heads), static_cast<int>(head_dim),
-                     positions, cos_table, sin_table, max_positions,
-                     static_cast<uint32_t>(wgs_per_row));
+  if (per_row > 0x7fffffff || rows > 0x7fffffffLL * kRopeThreads / per_row) return INT8KV_E_SHAPE;
+  const int64_t whole = kRopeThreads / per_row * per_row;  // (0 where a row has more chunks)
+  const int64_t step = whole >= kRopeThreads - kRopeThreads / 16 ? whole : kRopeThreads;
+  // (The kernel counts chunks in 31 bits; more than that take several launches.)
+  const int64_t most_rows = 0x7fffffff / per_row;
+  for (int64_t r0 = 0; r0 < rows; r0 += most_rows) {
+    const int64_t total = (rows - r0 < most_rows ? rows - r0 : most_rows) * per_row;
+    hipLaunchKernelGGL(rotary_kernel,
+                       dim3(static_cast<uint32_t>((total + step - 1) / step)), dim3(kRopeThreads), 0,
+                       static_cast<hipStream_t>(stream), static_cast<uint16_t*>(qkv) + r0 * row_stride, static_cast<uint32_t>(total),
+                       row_stride, static_cast<int>(head_dim), positions + r0, cos_table, sin_table,
+                       max_positions, static_cast<uint32_t>(step), static_cast<uint32_t>(per_row),
+                       divisor(static_cast<uint32_t>(per_row)),
+                       divisor(static_cast<uint32_t>(head_dim / 16)));
+  }
   return status(hipGetLastError());
 }
 

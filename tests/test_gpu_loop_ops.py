@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 import torch
 
+from int8kv import _lib
 from int8kv import decode_loop as DL
 
 pytestmark = pytest.mark.gpu
@@ -95,6 +96,34 @@ def test_rotary_inplace_bit_exact(cuda):
     x = qkv[4:, : heads * D].view(rows - 4, 1, heads, D)
     unfused = DL.apply_rope(x, cos[pos[4:]].view(rows - 4, 1, D), sin[pos[4:]].view(rows - 4, 1, D))
     assert torch.equal(got.cpu()[4:, : heads * D], unfused.reshape(rows - 4, heads * D))
+
+
+@pytest.mark.parametrize("rows,heads,d", [(5, 32, 128), (300, 33, 128), (41, 40, 64), (700, 3, 48), (17, 1, 16),
+                                          (129, 17, 256)])
+def test_rotary_rows_across_workgroups(cuda, rows, heads, d):
+    """Chunks per row below, at and above a workgroup's 256, rows that start inside one, strided rows."""
+    cos, sin = DL.rope_tables(DL.QwenShape(head_dim=d), 500, "cpu")
+    g = torch.Generator().manual_seed(rows)
+    qkv = (torch.randn(rows + 1, heads * d + 24, generator=g) * 4).to(torch.bfloat16)
+    pos = torch.randint(0, 500, (rows,), generator=g)
+    got = qkv.to(cuda)
+    DL.hip_rotary_(got[:rows], heads, d, pos.to(cuda), cos.to(cuda), sin.to(cuda))
+    x = qkv[:rows, : heads * d].view(rows, 1, heads, d)
+    ref = DL.apply_rope(x, cos[pos].view(rows, 1, d), sin[pos].view(rows, 1, d))
+    assert torch.equal(got.cpu()[:rows, : heads * d], ref.reshape(rows, heads * d))
+    assert torch.equal(got.cpu()[rows], qkv[rows]) and torch.equal(got.cpu()[:, heads * d :], qkv[:, heads * d :])
+
+
+def test_rotary_takes_the_widest_rows(cuda):
+    """2^30 chunks a row (34 GB each), so one launch per row: no row has a position in the table, so
+    none is touched."""
+    tables = torch.zeros(4, 16, device=cuda)
+    pos = torch.full((3,), -1, dtype=torch.int64, device=cuda)
+    status = _lib.load().int8kv_rotary_inplace(tables.data_ptr(), 3, 2**34, 2**30, 16, pos.data_ptr(),
+                                               tables.data_ptr(), tables.data_ptr(), 4,
+                                               _lib.stream_handle(cuda))
+    torch.cuda.synchronize()
+    assert status == 0 and not tables.any()
 
 
 @pytest.mark.parametrize("rows,ffn", [(32, 18944), (3, 1024), (1, 8)])
