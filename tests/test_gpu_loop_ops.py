@@ -269,7 +269,7 @@ def test_argmax_rows_matches_torch(cuda):
     assert out3[7].item() == 152_058 and out3[8].item() == 3 and out[9].item() == 20
 
 
-@pytest.mark.parametrize("vocab", [5, 8, 13, 8 * 1024, 8 * 8 * 1024 + 8, 152064])
+@pytest.mark.parametrize("vocab", [5, 8, 13, 8 * 1024, 8 * 1024 + 8, 16384, 16384 + 8, 32768 + 8, 8 * 8 * 1024 + 8, 152064])
 def test_argmax_rows_orders_special_values(cuda, vocab):
     """Rows that the comparison of whole vectors could get wrong: signed zeros and equal maxima in
     different vectors, all -inf, all negative, +inf, and NaN of either sign; one row per kind."""
