@@ -10,8 +10,9 @@
 // Mapping of 16-bit sources (wide kernels, head_dim % 16 == 0 and 16-byte aligned cache rows; fp32
 // sources and small calls take the row kernels, one 16-byte load per lane): grid.y = kv head,
 // one lane owns 16 consecutive head_dim elements of one (token, head) row of both K and V --
-// 32-byte source loads, 16-byte cache stores, 8 lanes per 128-element row.  The slot is read
-// first, so skipped rows cost no source bytes.  Sources are read and caches written with the
+// 32-byte source loads, 16-byte cache stores, 8 lanes per 128-element row.  The token-major
+// kernels, and the row kernels of calls above the Infinity Cache's size, read the slot first, so
+// skipped rows cost no source bytes there.  Sources are read and caches written with the
 // non-temporal hint: both are streamed once (262k-token write on MI355X: 193 -> 166 us, 4.2 ->
 // 4.9 TB/s).  Other layouts (head_dim % 16 == 8, or cache rows only 8-byte aligned) use the
 // narrow kernels: one lane per 8 elements, 8-byte stores.
@@ -22,7 +23,7 @@
 // consecutive lanes, and the dynamic write gathers four heads' scales into one 16-byte store
 // instead of four lone 4-byte stores (which cost a 32-byte write sector each: +23 % written
 // bytes at 262,144 tokens).  The dynamic write always uses it; the static write only when its
-// bytes exceed the Infinity Cache (static_token_major()).
+// bytes exceed the Infinity Cache (streams_past_cache()).
 //
 // The quotient x / scale is not divided per element: quantise() (int8kv_common.h) multiplies by
 // the correctly rounded reciprocal and divides only the elements whose quotient lies within
@@ -464,8 +465,10 @@ __global__ __launch_bounds__(256) void dynamic_write16_tm_kernel(DynWriteArgs d,
 // Row kernel of the dynamic write: vecs_per_row = head_dim / kPiece is a power of two of at most
 // 64, so a wave holds whole rows and the absmax butterfly stays inside the row.  Token-major, the
 // scales of four consecutive heads (when their lanes share a wave: vec_scales) leave in one
-// 16-byte store.
-template <int SRC, bool TM>
+// 16-byte store.  FIRST (calls above the Infinity Cache's size): a skipped row's source is not read,
+// for which the loads wait for the slot; else both are requested together (100,000 fp32 tokens x 4
+// x 128, no row skipped / every second: 97 / 71 us first, 94 / 80 together; 5,000: 7.2 and 6.9).
+template <int SRC, bool TM, bool FIRST>
 __global__ __launch_bounds__(256) void dynamic_write_rows_kernel(DynWriteArgs d, int lpr_shift, int lpt_shift) {
   const WriteArgs& a = d.w;
   constexpr int P = kPiece<SRC>;
@@ -473,17 +476,25 @@ __global__ __launch_bounds__(256) void dynamic_write_rows_kernel(DynWriteArgs d,
   uint32_t t;
   int h, dv;
   row_piece<TM>(a, lpr_shift, lpt_shift, t, h, dv);
-  // Every lane takes part in the exchanges; those past the last token and (token-major) of skipped
-  // rows hold zeros.
+  // The exchanges stay among one token's lanes, which leave together (FIRST) or all stay, with zeros
+  // past the last token.
   int64_t slot = -1;
   float x[P], y[P];
-#pragma unroll
-  for (int i = 0; i < P; ++i) x[i] = y[i] = 0.0f;
-  if ((int64_t)t < a.num_tokens) {
+  if constexpr (FIRST) {
+    if ((int64_t)t >= a.num_tokens) return;
     slot = load_index(a.slots, t, a.slots_is64);
-    if (slot >= a.capacity) slot = -1;
+    if (slot < 0 || slot >= a.capacity) return;
     load_piece<SRC>(a.key + ((int64_t)t * a.k_st + h * a.k_sh + P * dv) * esize, x);
     load_piece<SRC>(a.value + ((int64_t)t * a.v_st + h * a.v_sh + P * dv) * esize, y);
+  } else {
+#pragma unroll
+    for (int i = 0; i < P; ++i) x[i] = y[i] = 0.0f;
+    if ((int64_t)t < a.num_tokens) {
+      slot = load_index(a.slots, t, a.slots_is64);
+      if (slot >= a.capacity) slot = -1;
+      load_piece<SRC>(a.key + ((int64_t)t * a.k_st + h * a.k_sh + P * dv) * esize, x);
+      load_piece<SRC>(a.value + ((int64_t)t * a.v_st + h * a.v_sh + P * dv) * esize, y);
+    }
   }
   float km = 0.0f, vm = 0.0f;
 #pragma unroll
@@ -561,12 +572,12 @@ int token_major_shift(int64_t num_tokens, int32_t num_kv_heads, int32_t vecs_per
 }
 
 // The static write takes the token-major map only when it streams from HBM: its bytes exceed the
-// 256 MB Infinity Cache.  MI355X, 262,144 tokens (805 MB): 153.3-153.6 vs 157.2 us; 16,896 rows
+// 256 MB Infinity Cache (streams_past_cache).  MI355X, 262,144 tokens (805 MB): 153.3-153.6 vs 157.2 us; 16,896 rows
 // (50 MB, cache-resident): 13.1-13.2 vs 12.2 us.  The dynamic write always takes it (its scale
 // stores: 158-159 vs 175.7 us at 262,144 tokens, 13.7-14.0 vs 14.2-14.5 us at 16,896 rows).
 constexpr double kInfinityCacheBytes = 256.0 * 1024 * 1024;
 
-bool static_token_major(int64_t num_tokens, int32_t num_kv_heads, int32_t head_dim,
+bool streams_past_cache(int64_t num_tokens, int32_t num_kv_heads, int32_t head_dim,
                         int64_t src_esize) {
   return (double)num_tokens * num_kv_heads * head_dim * (2.0 * src_esize + 2.0) > kInfinityCacheBytes;
 }
@@ -593,14 +604,14 @@ int launch_rows(const WriteArgs& a, bool tm, dim3 grid, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-template <int SRC>
+template <int SRC, bool FIRST>
 int launch_dynamic_rows(const DynWriteArgs& d, bool tm, dim3 grid, hipStream_t s) {
   const int lpr_shift = __builtin_ctz((unsigned)d.w.vecs_per_row);
   if (tm)
-    hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, true>), grid, dim3(256), 0, s, d, lpr_shift,
+    hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, true, FIRST>), grid, dim3(256), 0, s, d, lpr_shift,
                        __builtin_ctz((unsigned)(d.w.vecs_per_row * d.w.num_kv_heads)));
   else
-    hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, false>), grid, dim3(256), 0, s, d, lpr_shift, 0);
+    hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, false, FIRST>), grid, dim3(256), 0, s, d, lpr_shift, 0);
   return (int)hipGetLastError();
 }
 
@@ -693,7 +704,7 @@ extern "C" int int8kv_cache_write(const void* key, const void* value, int src_dt
   const bool wide = wide_ok(key_cache, value_cache, key_cache_strides, value_cache_strides,
                             num_tokens, num_kv_heads, head_dim);
   const int64_t src_esize = src_dtype == INT8KV_F32 ? 4 : 2;
-  const bool streams = static_token_major(num_tokens, num_kv_heads, head_dim, src_esize);
+  const bool streams = streams_past_cache(num_tokens, num_kv_heads, head_dim, src_esize);
   if (wide && use_rows(src_dtype, num_tokens, num_kv_heads, head_dim)) {
     WriteArgs r = a;
     r.vecs_per_row = (int32_t)(head_dim * src_esize / 16);
@@ -801,10 +812,15 @@ extern "C" int int8kv_dynamic_cache_write(
       const bool tm = power_of_two(num_kv_heads);
       r.vec_scales = tm && scales_aligned && 4 * lpr <= kWave;
       dim3 grid;
-      if (rows_grid(r.w, tm, &grid))
-        return src_dtype == INT8KV_F32   ? launch_dynamic_rows<kF32>(r, tm, grid, s)
-               : src_dtype == INT8KV_F16 ? launch_dynamic_rows<kF16>(r, tm, grid, s)
-                                         : launch_dynamic_rows<kBF16>(r, tm, grid, s);
+      const bool first = streams_past_cache(num_tokens, num_kv_heads, head_dim,
+                                            src_dtype == INT8KV_F32 ? 4 : 2);
+      if (rows_grid(r.w, tm, &grid)) {
+        if (src_dtype == INT8KV_F32)
+          return first ? launch_dynamic_rows<kF32, true>(r, tm, grid, s)
+                       : launch_dynamic_rows<kF32, false>(r, tm, grid, s);
+        return src_dtype == INT8KV_F16 ? launch_dynamic_rows<kF16, false>(r, tm, grid, s)
+                                       : launch_dynamic_rows<kBF16, false>(r, tm, grid, s);
+      }
     }
   }
   if (wide && src_dtype != INT8KV_F32) {

@@ -16,7 +16,8 @@ pytestmark = pytest.mark.gpu
 # (tokens, kv heads, head_dim): one token; rows of 10 pieces; kv heads no power of two; more lanes
 # per token than a wave; 2^20 elements and one token fewer; fp32 past the Infinity Cache (256 MB).
 SHAPES = [(1, 4, 128), (37, 2, 80), (130, 3, 64), (63, 8, 256), (2047, 4, 128), (2048, 4, 128)]
-LARGE = [(60000, 4, 128)]
+LARGE = [(60000, 4, 128), (70000, 3, 128)]
+DTYPES = [torch.float32, torch.bfloat16, torch.float16]
 
 
 def _inputs(tokens, hkv, d, dtype, dev, seed):
@@ -31,11 +32,9 @@ def _inputs(tokens, hkv, d, dtype, dev, seed):
     return k, v, slots, torch.zeros(blocks, 16, hkv, d, dtype=torch.int8)
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
-@pytest.mark.parametrize("tokens,hkv,d", SHAPES + LARGE)
+@pytest.mark.parametrize("tokens,hkv,d,dtype", [(*s, t) for s in SHAPES for t in DTYPES]
+                         + [(*s, torch.float32) for s in LARGE])
 def test_static_write(cuda, tokens, hkv, d, dtype):
-    if tokens >= 60000 and dtype != torch.float32:
-        pytest.skip("16-bit sources of this size take the kernels tested elsewhere")
     k, v, slots, cache = _inputs(tokens, hkv, d, dtype, cuda, tokens + d)
     ks = torch.linspace(0.01, 0.08, hkv)
     vs = torch.linspace(0.03, 0.005, hkv)
@@ -49,8 +48,9 @@ def test_static_write(cuda, tokens, hkv, d, dtype):
 
 
 @pytest.mark.parametrize("strided_scales", [False, True])
-@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
-@pytest.mark.parametrize("tokens,hkv,d", [s for s in SHAPES if s[2] != 80] + [(40, 4, 512), (40, 4, 256)])
+@pytest.mark.parametrize("tokens,hkv,d,dtype", [
+    (*s, t) for s in [s for s in SHAPES if s[2] != 80] + [(40, 4, 512), (40, 4, 256)] for t in DTYPES[:2]]
+    + [(*s, torch.float32) for s in LARGE])
 def test_dynamic_write(cuda, tokens, hkv, d, dtype, strided_scales):
     k, v, slots, cache = _inputs(tokens, hkv, d, dtype, cuda, 3 * tokens + d)
     kc, vc = cache.to(cuda), cache.to(cuda)
