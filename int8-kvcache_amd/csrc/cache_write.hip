@@ -31,6 +31,8 @@
 // VALU instructions per element and made the write VALU-bound: 262,144 tokens 158 -> 155.6 us
 // static, 197 -> 175.6 us dynamic; 16,384 tokens 14.6 -> 12.1 us).
 
+#include <algorithm>
+
 #include "int8kv_common.h"
 
 namespace int8kv {
@@ -584,35 +586,55 @@ bool streams_past_cache(int64_t num_tokens, int32_t num_kv_heads, int32_t head_d
 
 bool power_of_two(int64_t n) { return n > 0 && (n & (n - 1)) == 0; }
 
-// Grid of a row kernel for `lpr` pieces per row (tm: the token-major map); false when the call's
-// pieces overflow its 32-bit index.
-bool rows_grid(const WriteArgs& a, bool tm, dim3* grid) {
-  const int64_t pieces = a.num_tokens * a.vecs_per_row * (tm ? a.num_kv_heads : 1);
-  if (pieces > 0x7fffff00LL) return false;
-  *grid = dim3((unsigned)((pieces + 255) / 256), tm ? 1u : (unsigned)a.num_kv_heads);
-  return true;
+// Launches a row kernel over all tokens, in as many calls as its 31-bit piece index takes (one up to
+// 2^31 pieces: 34 GB of K).  launch(token count, grid, first token).
+template <typename Launch>
+int for_rows(const WriteArgs& a, bool tm, Launch launch) {
+  const int64_t per_token = (int64_t)a.vecs_per_row * (tm ? a.num_kv_heads : 1);
+  const int64_t most = 0x7fffff00LL / per_token;
+  for (int64_t t0 = 0; t0 < a.num_tokens; t0 += most) {
+    const int64_t n = std::min(a.num_tokens - t0, most);
+    launch(n, dim3((unsigned)((n * per_token + 255) / 256), tm ? 1u : (unsigned)a.num_kv_heads), t0);
+  }
+  return (int)hipGetLastError();
+}
+
+// The arguments from token t0 on.
+template <int SRC>
+WriteArgs from_token(WriteArgs a, int64_t t0, int64_t n) {
+  constexpr int64_t esize = SRC == kF32 ? 4 : 2;
+  a.key += t0 * a.k_st * esize;
+  a.value += t0 * a.v_st * esize;
+  a.slots = static_cast<const char*>(a.slots) + t0 * (a.slots_is64 ? 8 : 4);
+  a.num_tokens = n;
+  return a;
 }
 
 template <int SRC>
-int launch_rows(const WriteArgs& a, bool tm, dim3 grid, hipStream_t s) {
-  if (tm)
-    hipLaunchKernelGGL((cache_write_rows_kernel<SRC, true>), grid, dim3(256), 0, s, a,
-                       __builtin_ctz((unsigned)a.vecs_per_row),
-                       __builtin_ctz((unsigned)(a.vecs_per_row * a.num_kv_heads)));
-  else
-    hipLaunchKernelGGL((cache_write_rows_kernel<SRC, false>), grid, dim3(256), 0, s, a, 0, 0);
-  return (int)hipGetLastError();
+int launch_rows(const WriteArgs& a, bool tm, hipStream_t s) {
+  return for_rows(a, tm, [&](int64_t n, dim3 grid, int64_t t0) {
+    const WriteArgs c = from_token<SRC>(a, t0, n);
+    if (tm)
+      hipLaunchKernelGGL((cache_write_rows_kernel<SRC, true>), grid, dim3(256), 0, s, c,
+                         __builtin_ctz((unsigned)a.vecs_per_row),
+                         __builtin_ctz((unsigned)(a.vecs_per_row * a.num_kv_heads)));
+    else
+      hipLaunchKernelGGL((cache_write_rows_kernel<SRC, false>), grid, dim3(256), 0, s, c, 0, 0);
+  });
 }
 
 template <int SRC, bool FIRST>
-int launch_dynamic_rows(const DynWriteArgs& d, bool tm, dim3 grid, hipStream_t s) {
+int launch_dynamic_rows(const DynWriteArgs& d, bool tm, hipStream_t s) {
   const int lpr_shift = __builtin_ctz((unsigned)d.w.vecs_per_row);
-  if (tm)
-    hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, true, FIRST>), grid, dim3(256), 0, s, d, lpr_shift,
-                       __builtin_ctz((unsigned)(d.w.vecs_per_row * d.w.num_kv_heads)));
-  else
-    hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, false, FIRST>), grid, dim3(256), 0, s, d, lpr_shift, 0);
-  return (int)hipGetLastError();
+  return for_rows(d.w, tm, [&](int64_t n, dim3 grid, int64_t t0) {
+    DynWriteArgs c = d;
+    c.w = from_token<SRC>(d.w, t0, n);
+    if (tm)
+      hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, true, FIRST>), grid, dim3(256), 0, s, c, lpr_shift,
+                         __builtin_ctz((unsigned)(d.w.vecs_per_row * d.w.num_kv_heads)));
+    else
+      hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, false, FIRST>), grid, dim3(256), 0, s, c, lpr_shift, 0);
+  });
 }
 
 // Whether a call takes the row kernels.
@@ -708,14 +730,13 @@ extern "C" int int8kv_cache_write(const void* key, const void* value, int src_dt
   if (wide && use_rows(src_dtype, num_tokens, num_kv_heads, head_dim)) {
     WriteArgs r = a;
     r.vecs_per_row = (int32_t)(head_dim * src_esize / 16);
-    const bool tm = streams && power_of_two(num_kv_heads) && power_of_two(r.vecs_per_row);
-    dim3 grid;
-    if (rows_grid(r, tm, &grid))
-      return src_dtype == INT8KV_F32   ? launch_rows<kF32>(r, tm, grid, s)
-             : src_dtype == INT8KV_F16 ? launch_rows<kF16>(r, tm, grid, s)
-                                       : launch_rows<kBF16>(r, tm, grid, s);
+    const bool tm = streams && power_of_two(num_kv_heads) && power_of_two(r.vecs_per_row) &&
+                    (int64_t)r.vecs_per_row * num_kv_heads <= 1 << 24;  // (a token in a 31-bit index)
+    return src_dtype == INT8KV_F32   ? launch_rows<kF32>(r, tm, s)
+           : src_dtype == INT8KV_F16 ? launch_rows<kF16>(r, tm, s)
+                                     : launch_rows<kBF16>(r, tm, s);
   }
-  if (wide && src_dtype != INT8KV_F32) {
+  if (wide) {  // (fp32 sources took the row kernels)
     a.vecs_per_row = head_dim / 16;
     const int lpt_shift = token_major_shift(num_tokens, num_kv_heads, a.vecs_per_row);
     if (lpt_shift >= 0 && streams) {
@@ -811,16 +832,13 @@ extern "C" int int8kv_dynamic_cache_write(
       r.w.vecs_per_row = lpr;
       const bool tm = power_of_two(num_kv_heads);
       r.vec_scales = tm && scales_aligned && 4 * lpr <= kWave;
-      dim3 grid;
       const bool first = streams_past_cache(num_tokens, num_kv_heads, head_dim,
                                             src_dtype == INT8KV_F32 ? 4 : 2);
-      if (rows_grid(r.w, tm, &grid)) {
-        if (src_dtype == INT8KV_F32)
-          return first ? launch_dynamic_rows<kF32, true>(r, tm, grid, s)
-                       : launch_dynamic_rows<kF32, false>(r, tm, grid, s);
-        return src_dtype == INT8KV_F16 ? launch_dynamic_rows<kF16, false>(r, tm, grid, s)
-                                       : launch_dynamic_rows<kBF16, false>(r, tm, grid, s);
-      }
+      if (src_dtype == INT8KV_F32)
+        return first ? launch_dynamic_rows<kF32, true>(r, tm, s)
+                     : launch_dynamic_rows<kF32, false>(r, tm, s);
+      return src_dtype == INT8KV_F16 ? launch_dynamic_rows<kF16, false>(r, tm, s)
+                                     : launch_dynamic_rows<kBF16, false>(r, tm, s);
     }
   }
   if (wide && src_dtype != INT8KV_F32) {
