@@ -275,6 +275,68 @@ def test_groups_above_16_spread_over_waves(cuda, hq, hkv, d, batch, tokens, per_
     _check(out, ref, f"{cache} {hq}/{hkv} d={d} {batch}x{tokens}")
 
 
+@pytest.mark.parametrize("cache", ["int8", "fp16"])
+@pytest.mark.parametrize("hq,d,block", [(71, 64, 32), (71, 64, 256), (48, 128, 64), (40, 80, 16)])
+def test_groups_above_16_views(cuda, hq, d, block, cache):
+    """64-bit tables and lengths, tables, queries, caches and outputs that are views into wider
+    tensors, blocks of other sizes, fp16 queries: column tiles shared by a wave as for plain tensors."""
+    lens = [5000, 0, 700, 4097, 1, 2222, 4999, 31] + [3000 + 11 * i for i in range(12)]
+    c = decode_case(lens, seed=hq + block, hq=hq, hkv=1, head_dim=d, block_size=block, extra_blocks=3)
+    q, kc, vc, bt, sl, ks, vs = to_dev(c, cuda)
+    assert plan_columns(torch.int8 if cache == "int8" else torch.float16, len(lens), hq, 1, d,
+                        bt.shape[1], bs=block)[0] >= 2
+    if cache == "fp16":
+        k_cpu, v_cpu = bf16_caches(c, torch.float16)
+        kc, vc = k_cpu.to(cuda), v_cpu.to(cuda)
+        ref = O.paged_attention_ref(c.query.float().numpy(), k_cpu.float().numpy(),
+                                    v_cpu.float().numpy(), c.block_tables.numpy(), c.seq_lens.numpy())
+    else:
+        ref = oracle_int8(c)
+    kv = torch.stack([kc, vc], dim=1)  # [blocks, 2, block, 1, d]: K and V of a block side by side
+    kc, vc = kv[:, 0], kv[:, 1]
+    tables = torch.full((len(lens), 2 * bt.shape[1]), -5, dtype=torch.int64, device=cuda)
+    tables[:, ::2] = bt
+    query = torch.full((len(lens), hq + 2, d + 16), float("nan"), dtype=torch.float16, device=cuda)
+    query[:, 1 : hq + 1, :d] = q.to(torch.float16)
+    out = torch.full_like(query, 7.0)
+    view = out[:, 1 : hq + 1, :d]
+    _decode.paged_decode(query[:, 1 : hq + 1, :d], kc, vc, tables[:, ::2], sl.to(torch.int64),
+                         ks if cache == "int8" else None, vs if cache == "int8" else None, view)
+    torch.cuda.synchronize()
+    _check(view, ref, f"{cache} {hq}/1 d={d} block {block}")
+    view.fill_(7.0)
+    assert (out == 7).all(), "written outside the output view"
+
+
+@pytest.mark.parametrize("cache", ["int8", "bf16"])
+def test_groups_above_16_non_finite_queries(cuda, cache):
+    """A NaN, an infinity of either sign and a huge finite query row: the rows of those heads as one wave
+    per tile gives them, all others untouched by them."""
+    lens = [4096] * 20 + [17, 0]
+    c = decode_case(lens, seed=77, hq=71, hkv=1, head_dim=64)
+    q, kc, vc, bt, sl, ks, vs = to_dev(c, cuda)
+    if cache == "bf16":
+        kc, vc = (t.to(cuda) for t in bf16_caches(c))
+        ks = vs = None
+    plain = torch.empty_like(q)
+    _decode.paged_decode(q, kc, vc, bt, sl, ks, vs, plain)
+    bad = q.clone()
+    bad[0, 3, 5], bad[1, 20, 1], bad[2, 70, 0], bad[3, 40] = float("nan"), float("inf"), float("-inf"), 3e38
+    touched = torch.zeros(len(lens), 71, dtype=torch.bool, device=cuda)
+    touched[0, 3] = touched[1, 20] = touched[2, 70] = touched[3, 40] = True
+    out = torch.empty_like(q)
+    _decode.paged_decode(bad, kc, vc, bt, sl, ks, vs, out)
+    assert torch.equal(out[~touched], plain[~touched])
+    # The same heads as groups of 16 or fewer: one wave per tile.
+    for b, h in touched.nonzero().tolist():
+        one = torch.empty(1, 1, 64, dtype=q.dtype, device=cuda)
+        _decode.paged_decode(bad[b : b + 1, h : h + 1], kc, vc, bt[b : b + 1], sl[b : b + 1], ks, vs, one)
+        assert torch.equal(torch.isnan(one[0, 0]), torch.isnan(out[b, h])), (b, h)
+        same = one[0, 0] == out[b, h]
+        near = (one[0, 0].float() - out[b, h].float()).abs() <= MAX_ABS
+        assert (same | near | torch.isnan(one[0, 0])).all(), (b, h)
+
+
 def test_groups_above_16_with_the_automatic_counts_workspace(cuda):
     """71 heads on one kv head at 64: a workspace of the automatic count's ranges (those of 5 kv
     heads), of any more, and one byte too few."""

@@ -2,7 +2,8 @@
 against the separate kernels bit for bit.
 
 Bound of a product: fp32 sums of K exact bf16 products in any order are within K 2^-24 sum|x w| of
-the exact sum, and the bf16 result within half a spacing (2^-8 relative, safely) of that.
+the exact sum, and the bf16 result within half a spacing (2^-8 relative, safely) of that.  It is the worst
+case, far above the errors of a correct sum: test_exact_sums holds them to none.
 """
 
 from __future__ import annotations
@@ -41,6 +42,26 @@ def test_linear_matches_float64(cuda, rows, k, n):
         err = (out[:rows].double() - ref).abs()
         assert (err <= 2.0**-8 * ref.abs() + k * 2.0**-24 * (mass + ref.abs())).all()
         assert torch.isnan(out[rows]).all(), "a row past x was written"
+
+
+@pytest.mark.parametrize("rows", [1, 17, 32])
+@pytest.mark.parametrize("k,n", [(64, 16), (2624, 48), (4096, 64), (4160, 64), (18944, 3584), (32768, 32)])
+def test_exact_sums(cuda, rows, k, n):
+    """Whole numbers whose products and sums fp32 holds exactly (at most 8 x 4 x K < 2^24): the
+    result is the exact sum rounded to bf16, whatever the order; a column of K left out or a partial sum
+    kept in fewer bits changes it.  The fused residual add sums the same way."""
+    g = torch.Generator(device=cuda).manual_seed(rows + k)
+    x = torch.randint(-8, 9, (rows, k), generator=g, device=cuda).to(torch.bfloat16)
+    w = torch.randint(-4, 5, (n, k), generator=g, device=cuda).to(torch.bfloat16)
+    b = torch.randint(-64, 65, (n,), generator=g, device=cuda).to(torch.bfloat16)
+    work = torch.empty(max(DL.linear_workspace_bytes(rows, w), 16), dtype=torch.uint8, device=cuda)
+    out = torch.empty(rows, n, dtype=torch.bfloat16, device=cuda)
+    exact = x.double() @ w.double().t()
+    assert torch.equal(DL.hip_linear(x, w, b, out, work), (exact + b.double()).to(torch.bfloat16))
+    residual = torch.randint(-100, 101, (rows, n), generator=g, device=cuda).to(torch.bfloat16)
+    want = (residual.double() + exact.to(torch.bfloat16).double()).to(torch.bfloat16)
+    DL.hip_linear_add_rms_norm(x, w, residual, torch.ones_like(b), torch.empty_like(out), 1e-6, work)
+    assert torch.equal(residual, want)
 
 
 @pytest.mark.parametrize("rows", [1, 16, 32])
