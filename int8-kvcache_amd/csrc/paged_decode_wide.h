@@ -4,11 +4,12 @@
 //
 // Bound: with one wave per column tile (decode_kernel's layout) every tile of 16 heads read,
 // dequantised and multiplied its kv head's K/V again, and 71 heads on one kv head took 5 waves'
-// time for one wave's bytes (head_dim 64, INT8, B = 40 x 4096, 21.7 MB: 41.2 us per call, 0.53
+// time for one wave's bytes (head_dim 64, INT8, B = 40 x 4096, 21.7 MB: 40.4 us per call, 0.54
 // TB/s).  Here the tile's K and V operands are built once and serve all CT tiles; what is left
 // per extra tile is its MFMAs and its softmax (per 32 tokens and wave 0.43 + 0.29 CT us, against
-// 1.04 us per wave and tile): 28.5 us per call, bound by that arithmetic and by ~12 us from the
-// launch to a range's first tile and from its last tile to its records.
+// 1.04 us per wave and tile): 27.3 us per call, bound by that arithmetic and by ~12 us from the
+// launch to a range's first tile and from its last tile to its records.  How many tiles a wave
+// takes, and which calls keep one wave per tile: wide_column_tiles (paged_decode.hip).
 // Split: a range of the token stream (the plan of decode_kernel) belongs to a workgroup of four
 // waves, one per SIMD, which share each of its sequences' tiles and combine their softmax states
 // in LDS.  One wave per range instead would leave four times the partial records, and a record

@@ -8,8 +8,9 @@ namespace int8kv_loop {
 
 // silu(g) = g / (1 + exp(-g)) without expf's range handling and the IEEE divide (about 35
 // instructions an element, in branches whose registers the fused product does not have):
-// -g log2(e) as a rounded product plus its rounding error, the error applied to exp2 of the
-// product; the reciprocal refined once and the quotient corrected by its remainder.  Over every
+// -g log2(e) as a rounded product plus its rounding error (Cody and Waite's split constant), the
+// error applied to exp2 of the product; the hardware's reciprocal refined by one Newton-Raphson
+// step and the quotient corrected by its remainder (Markstein).  Over every
 // bf16 value with |g| < 87 the result is within 1.35e-7 relative of 64 bits, which is also what
 // a correctly rounded exp and divide give.
 constexpr float kLog2eHi = 1.44269502162933349609375f;  // log2(e) rounded to fp32, and the rest

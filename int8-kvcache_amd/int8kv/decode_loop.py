@@ -64,7 +64,9 @@ FUSED_STEP = True
 MODES = ("int8", "bf16")
 
 # hipBLASLt solutions chosen by torch's TunableOp for the decode step's GEMMs (M = batch rows)
-# on MI355X; written by ``configure_gemm_tuning("tune", ...)`` and read back with "use".
+# on MI355X; written by ``configure_gemm_tuning("tune", ...)`` and read back with "use".  Its entries
+# are the 32-row shapes of Qwen2.5-7B, which a step reaches only where the library's own products
+# do not run (DecodeLoop._skinny).
 GEMM_TUNING_FILE = Path(__file__).resolve().parent / "gemm_tuning_mi355x.csv"
 GEMM_TUNING_MODES = ("off", "use", "tune")
 
