@@ -11,8 +11,8 @@
 // sources and small calls take the row kernels, one 16-byte load per lane): grid.y = kv head,
 // one lane owns 16 consecutive head_dim elements of one (token, head) row of both K and V --
 // 32-byte source loads, 16-byte cache stores, 8 lanes per 128-element row.  The token-major
-// kernels, and the row kernels of calls above the Infinity Cache's size, read the slot first, so
-// skipped rows cost no source bytes there.  Sources are read and caches written with the
+// kernels, the static row kernel above the Infinity Cache's size and the dynamic one above half of
+// it, read the slot first, so skipped rows cost no source bytes there.  Sources are read and caches written with the
 // non-temporal hint: both are streamed once (262k-token write on MI355X: 193 -> 166 us, 4.2 ->
 // 4.9 TB/s).  Other layouts (head_dim % 16 == 8, or cache rows only 8-byte aligned) use the
 // narrow kernels: one lane per 8 elements, 8-byte stores.
@@ -464,40 +464,17 @@ __global__ __launch_bounds__(256) void dynamic_write16_tm_kernel(DynWriteArgs d,
   }
 }
 
-// Row kernel of the dynamic write: vecs_per_row = head_dim / kPiece is a power of two of at most
+// Row kernels of the dynamic write: vecs_per_row = head_dim / kPiece is a power of two of at most
 // 64, so a wave holds whole rows and the absmax butterfly stays inside the row.  Token-major, the
 // scales of four consecutive heads (when their lanes share a wave: vec_scales) leave in one
-// 16-byte store.  FIRST (calls above the Infinity Cache's size): a skipped row's source is not read,
-// for which the loads wait for the slot; else both are requested together (100,000 fp32 tokens x 4
-// x 128, no row skipped / every second: 97 / 71 us first, 94 / 80 together; 5,000: 7.2 and 6.9).
-template <int SRC, bool TM, bool FIRST>
-__global__ __launch_bounds__(256) void dynamic_write_rows_kernel(DynWriteArgs d, int lpr_shift, int lpt_shift) {
+// 16-byte store.
+
+// A row's scales and codes from its lanes' pieces, which all come here (slot < 0: for the exchanges only).
+template <int P, bool TM>
+__device__ __forceinline__ void write_dynamic_piece(const DynWriteArgs& d, const float (&x)[P],
+                                                    const float (&y)[P], int64_t slot, int h, int dv,
+                                                    int lpr_shift) {
   const WriteArgs& a = d.w;
-  constexpr int P = kPiece<SRC>;
-  constexpr int esize = SRC == kF32 ? 4 : 2;
-  uint32_t t;
-  int h, dv;
-  row_piece<TM>(a, lpr_shift, lpt_shift, t, h, dv);
-  // The exchanges stay among one token's lanes, which leave together (FIRST) or all stay, with zeros
-  // past the last token.
-  int64_t slot = -1;
-  float x[P], y[P];
-  if constexpr (FIRST) {
-    if ((int64_t)t >= a.num_tokens) return;
-    slot = load_index(a.slots, t, a.slots_is64);
-    if (slot < 0 || slot >= a.capacity) return;
-    load_piece<SRC>(a.key + ((int64_t)t * a.k_st + h * a.k_sh + P * dv) * esize, x);
-    load_piece<SRC>(a.value + ((int64_t)t * a.v_st + h * a.v_sh + P * dv) * esize, y);
-  } else {
-#pragma unroll
-    for (int i = 0; i < P; ++i) x[i] = y[i] = 0.0f;
-    if ((int64_t)t < a.num_tokens) {
-      slot = load_index(a.slots, t, a.slots_is64);
-      if (slot >= a.capacity) slot = -1;
-      load_piece<SRC>(a.key + ((int64_t)t * a.k_st + h * a.k_sh + P * dv) * esize, x);
-      load_piece<SRC>(a.value + ((int64_t)t * a.v_st + h * a.v_sh + P * dv) * esize, y);
-    }
-  }
   float km = 0.0f, vm = 0.0f;
 #pragma unroll
   for (int i = 0; i < P; ++i) {
@@ -541,6 +518,69 @@ __global__ __launch_bounds__(256) void dynamic_write_rows_kernel(DynWriteArgs d,
     *kp = ks;
     *vp = vs;
   }
+}
+
+// One piece per lane, its slot and source requested together.
+template <int SRC, bool TM>
+__global__ __launch_bounds__(256) void dynamic_write_rows_kernel(DynWriteArgs d, int lpr_shift, int lpt_shift) {
+  const WriteArgs& a = d.w;
+  constexpr int P = kPiece<SRC>;
+  constexpr int esize = SRC == kF32 ? 4 : 2;
+  uint32_t t;
+  int h, dv;
+  row_piece<TM>(a, lpr_shift, lpt_shift, t, h, dv);
+  // Every lane takes part in the exchanges; those past the last token hold zeros.
+  int64_t slot = -1;
+  float x[P], y[P];
+#pragma unroll
+  for (int i = 0; i < P; ++i) x[i] = y[i] = 0.0f;
+  if ((int64_t)t < a.num_tokens) {
+    slot = load_index(a.slots, t, a.slots_is64);
+    if (slot >= a.capacity) slot = -1;
+    load_piece<SRC>(a.key + ((int64_t)t * a.k_st + h * a.k_sh + P * dv) * esize, x);
+    load_piece<SRC>(a.value + ((int64_t)t * a.v_st + h * a.v_sh + P * dv) * esize, y);
+  }
+  write_dynamic_piece<P, TM>(d, x, y, slot, h, dv, lpr_shift);
+}
+
+// Large token-major calls of fp32 sources (kStreamedBytes): the slot first, so that a skipped row's
+// source is not read, and per lane the same piece of kStreamTokens tokens, `apart` from each other,
+// whose slots and then sources are requested together, since one piece alone leaves the memory
+// idle while its slot is on the way (5 % slower).  us with no row / every second row skipped, this and the
+// kernel above: 100,000 tokens x 4 x 128 94 / 56 and 94 / 79; 32,000 (164 MB) 32.7 / 20.6 and 32.2 /
+// 25.8; 16,000 (82 MB) 18.4 / 12.1 and 17.5 / 14.2, 4,000 6.5 / 5.4 and 5.8 / 5.2.  Head-major calls lose
+// 4 % with no row skipped and keep the kernel above.
+constexpr int kStreamTokens = 2;
+constexpr double kStreamedBytes = 128.0 * 1024 * 1024;
+
+__global__ __launch_bounds__(256) void dynamic_write_streamed_kernel(DynWriteArgs d, int lpr_shift, int lpt_shift,
+                                                                     uint32_t apart) {
+  const WriteArgs& a = d.w;
+  constexpr int P = kPiece<kF32>;
+  uint32_t t0;
+  int h, dv;
+  row_piece<true>(a, lpr_shift, lpt_shift, t0, h, dv);
+  if (t0 >= apart) return;
+  int64_t slot[kStreamTokens];
+#pragma unroll
+  for (int j = 0; j < kStreamTokens; ++j) {
+    const int64_t t = t0 + (int64_t)j * apart;
+    slot[j] = t < a.num_tokens ? load_index(a.slots, t, a.slots_is64) : -1;
+    if (slot[j] >= a.capacity) slot[j] = -1;
+  }
+  float x[kStreamTokens][P], y[kStreamTokens][P];
+#pragma unroll
+  for (int j = 0; j < kStreamTokens; ++j) {
+    const int64_t t = t0 + (int64_t)j * apart;
+    if (slot[j] >= 0) {
+      load_piece<kF32>(a.key + (t * a.k_st + h * a.k_sh + P * dv) * 4, x[j]);
+      load_piece<kF32>(a.value + (t * a.v_st + h * a.v_sh + P * dv) * 4, y[j]);
+    }
+  }
+  // (A token's lanes hold the same slots and stay together in each exchange.)
+#pragma unroll
+  for (int j = 0; j < kStreamTokens; ++j)
+    if (slot[j] >= 0) write_dynamic_piece<P, true>(d, x[j], y[j], slot[j], h, dv, lpr_shift);
 }
 
 }  // namespace int8kv
@@ -587,15 +627,16 @@ bool streams_past_cache(int64_t num_tokens, int32_t num_kv_heads, int32_t head_d
 bool power_of_two(int64_t n) { return n > 0 && (n & (n - 1)) == 0; }
 
 // Launches a row kernel over all tokens, in as many calls as its 31-bit piece index takes (one up to
-// 2^31 pieces: 34 GB of K).  launch(token count, grid, first token).
+// 2^31 pieces: 34 GB of K).  launch(token count, grid for n tokens, first token).
 template <typename Launch>
 int for_rows(const WriteArgs& a, bool tm, Launch launch) {
   const int64_t per_token = (int64_t)a.vecs_per_row * (tm ? a.num_kv_heads : 1);
   const int64_t most = 0x7fffff00LL / per_token;
-  for (int64_t t0 = 0; t0 < a.num_tokens; t0 += most) {
-    const int64_t n = std::min(a.num_tokens - t0, most);
-    launch(n, dim3((unsigned)((n * per_token + 255) / 256), tm ? 1u : (unsigned)a.num_kv_heads), t0);
-  }
+  const auto grid = [&](int64_t n) {
+    return dim3((unsigned)((n * per_token + 255) / 256), tm ? 1u : (unsigned)a.num_kv_heads);
+  };
+  for (int64_t t0 = 0; t0 < a.num_tokens; t0 += most)
+    launch(std::min(a.num_tokens - t0, most), grid, t0);
   return (int)hipGetLastError();
 }
 
@@ -612,28 +653,40 @@ WriteArgs from_token(WriteArgs a, int64_t t0, int64_t n) {
 
 template <int SRC>
 int launch_rows(const WriteArgs& a, bool tm, hipStream_t s) {
-  return for_rows(a, tm, [&](int64_t n, dim3 grid, int64_t t0) {
+  return for_rows(a, tm, [&](int64_t n, auto grid, int64_t t0) {
     const WriteArgs c = from_token<SRC>(a, t0, n);
     if (tm)
-      hipLaunchKernelGGL((cache_write_rows_kernel<SRC, true>), grid, dim3(256), 0, s, c,
+      hipLaunchKernelGGL((cache_write_rows_kernel<SRC, true>), grid(n), dim3(256), 0, s, c,
                          __builtin_ctz((unsigned)a.vecs_per_row),
                          __builtin_ctz((unsigned)(a.vecs_per_row * a.num_kv_heads)));
     else
-      hipLaunchKernelGGL((cache_write_rows_kernel<SRC, false>), grid, dim3(256), 0, s, c, 0, 0);
+      hipLaunchKernelGGL((cache_write_rows_kernel<SRC, false>), grid(n), dim3(256), 0, s, c, 0, 0);
   });
 }
 
-template <int SRC, bool FIRST>
+template <int SRC>
 int launch_dynamic_rows(const DynWriteArgs& d, bool tm, hipStream_t s) {
   const int lpr_shift = __builtin_ctz((unsigned)d.w.vecs_per_row);
-  return for_rows(d.w, tm, [&](int64_t n, dim3 grid, int64_t t0) {
+  const int lpt_shift = tm ? __builtin_ctz((unsigned)(d.w.vecs_per_row * d.w.num_kv_heads)) : 0;
+  return for_rows(d.w, tm, [&](int64_t n, auto grid, int64_t t0) {
     DynWriteArgs c = d;
     c.w = from_token<SRC>(d.w, t0, n);
     if (tm)
-      hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, true, FIRST>), grid, dim3(256), 0, s, c, lpr_shift,
-                         __builtin_ctz((unsigned)(d.w.vecs_per_row * d.w.num_kv_heads)));
+      hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, true>), grid(n), dim3(256), 0, s, c, lpr_shift, lpt_shift);
     else
-      hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, false, FIRST>), grid, dim3(256), 0, s, c, lpr_shift, 0);
+      hipLaunchKernelGGL((dynamic_write_rows_kernel<SRC, false>), grid(n), dim3(256), 0, s, c, lpr_shift, lpt_shift);
+  });
+}
+
+int launch_dynamic_streamed(const DynWriteArgs& d, hipStream_t s) {
+  const int lpr_shift = __builtin_ctz((unsigned)d.w.vecs_per_row);
+  const int lpt_shift = __builtin_ctz((unsigned)(d.w.vecs_per_row * d.w.num_kv_heads));
+  return for_rows(d.w, true, [&](int64_t n, auto grid, int64_t t0) {
+    DynWriteArgs c = d;
+    c.w = from_token<kF32>(d.w, t0, n);
+    const int64_t apart = (n + kStreamTokens - 1) / kStreamTokens;
+    hipLaunchKernelGGL(dynamic_write_streamed_kernel, grid(apart), dim3(256), 0, s, c, lpr_shift, lpt_shift,
+                       (uint32_t)apart);
   });
 }
 
@@ -832,13 +885,12 @@ extern "C" int int8kv_dynamic_cache_write(
       r.w.vecs_per_row = lpr;
       const bool tm = power_of_two(num_kv_heads);
       r.vec_scales = tm && scales_aligned && 4 * lpr <= kWave;
-      const bool first = streams_past_cache(num_tokens, num_kv_heads, head_dim,
-                                            src_dtype == INT8KV_F32 ? 4 : 2);
       if (src_dtype == INT8KV_F32)
-        return first ? launch_dynamic_rows<kF32, true>(r, tm, s)
-                     : launch_dynamic_rows<kF32, false>(r, tm, s);
-      return src_dtype == INT8KV_F16 ? launch_dynamic_rows<kF16, false>(r, tm, s)
-                                     : launch_dynamic_rows<kBF16, false>(r, tm, s);
+        return tm && (double)num_tokens * num_kv_heads * head_dim * 10.0 > kStreamedBytes
+                   ? launch_dynamic_streamed(r, s)
+                   : launch_dynamic_rows<kF32>(r, tm, s);
+      return src_dtype == INT8KV_F16 ? launch_dynamic_rows<kF16>(r, tm, s)
+                                     : launch_dynamic_rows<kBF16>(r, tm, s);
     }
   }
   if (wide && src_dtype != INT8KV_F32) {

@@ -16,9 +16,10 @@ from oracle import int8kv_oracle as O
 pytestmark = pytest.mark.gpu
 
 # (tokens, kv heads, head_dim): one token; rows of 10 pieces; kv heads no power of two; more lanes
-# per token than a wave; 2^20 elements and one token fewer; fp32 past the Infinity Cache (256 MB).
+# per token than a wave; 2^20 elements and one token fewer; fp32 past the Infinity Cache
+# (256 MB) and on both sides of half of it, odd token counts among them.
 SHAPES = [(1, 4, 128), (37, 2, 80), (130, 3, 64), (63, 8, 256), (2047, 4, 128), (2048, 4, 128)]
-LARGE = [(60000, 4, 128), (70000, 3, 128)]
+LARGE = [(60000, 4, 128), (70000, 3, 128), (26215, 4, 128), (13107, 8, 128)]
 DTYPES = [torch.float32, torch.bfloat16, torch.float16]
 
 
