@@ -183,3 +183,18 @@ def test_oversized_request_is_refused(cuda):
         _noalloc(q, kc, vc, bt, sl, ks, vs, out, (16 << 20) // per_range + 1)
     torch.cuda.synchronize()
     assert not out.any()  # nothing was launched
+
+
+@pytest.mark.parametrize("hq,d,ranges", [(71, 64, 0), (71, 64, 300), (128, 128, 0), (256, 128, 0), (48, 112, 0)])
+def test_groups_above_16_sharing_operands(cuda, hq, d, ranges):
+    """Several column tiles per wave: the ranges launched fit the scratch (71 heads at 64: more than
+    the automatic count; 256 at 128: the scratch holds 62 ranges) and give the same bits."""
+    lens = [4096 - 3 * i for i in range(40)]
+    c = decode_case(lens, seed=hq + d, hq=hq, hkv=1, head_dim=d)
+    q, kc, vc, bt, sl, ks, vs = to_dev(c, cuda)
+    want = _with_workspace(q, kc, vc, bt, sl, ks, vs, ranges)
+    got = _noalloc(q, kc, vc, bt, sl, ks, vs, torch.full_like(q, float("nan")), ranges)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    err, cos, _ = metrics(got.float().cpu().numpy(), oracle_int8(c))
+    assert err <= MAX_ABS and cos >= MIN_COS, (err, cos)
